@@ -666,7 +666,7 @@ int dcq_kv_attention(int cache_type, const void* k_arena, const void* v_arena, i
         !aligned(block_table, 4))
         return DCQ_ERR_MISALIGNED;
     if (q_stride_bytes % 16 || kv_stride_bytes % 16 || out_stride_bytes % 4) return DCQ_ERR_MISALIGNED;
-    const size_t need = attn_workspace_bytes(head_dim, n_head, n_head_kv, (int)n_tokens, (int)n_past);
+    const size_t need = attn_workspace_min_bytes(head_dim, n_head, n_head_kv, (int)n_tokens, (int)n_past);
     if (need) {
         if (!workspace || workspace_bytes < need) return DCQ_ERR_WORKSPACE;
         if (!aligned(workspace, 256)) return DCQ_ERR_MISALIGNED;

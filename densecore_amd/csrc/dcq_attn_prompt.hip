@@ -1,0 +1,419 @@
+// dcq_attn_prompt.hip — attention of prompts and prompt chunks over the paged KV cache, on f16 MFMA.
+//
+// The reference's standard attention path (core/src/inference.cpp:1577-1746) in fp32, for calls with
+// many query rows; decode-sized calls keep attn_kernel (dcq_kv.hip). The fp32 MFMA peak is 157
+// TFLOP/s, a sixteenth of the f16 one, so each fp32 operand x is split into two f16 pieces,
+//   x = 2^e (h + l),  h = f16(x 2^-e),  l = f16(x 2^-e - h)   (round to nearest even)
+// and a product takes three MFMAs: h h' + h l' + l h'. Two pieces hold 22 bits or more of x, and the
+// dropped l l' is below 2^-22 of the product. The exponents keep the pieces in f16's range for every fp32
+// input: one per query row, and one per 8 keys for K and for V (the wave that stages 8 keys finds
+// their largest magnitude), chosen so that the largest magnitude lands in [2^14, 2^15). Elements down
+// to 2^-16 of it still have a normal l.
+//
+// Work split. The query rows of a KV head are the (token, query head of its group) pairs, token-major,
+// so any group size fills the tiles: a workgroup takes 128 consecutive rows, each of its 4 waves 32 of
+// them (one column of MFMA tiles), and walks the keys its rows see in blocks of 32, double-buffered in
+// LDS. The staging of a block (loads, exponents, split) is shared by the 128 rows; its loads are issued
+// before the previous block's MFMAs and its conversion runs after them.
+//   S^T = K Q^T (keys x rows): A = K pieces (16-byte LDS reads), B = Q pieces (registers). Lane l then
+//   holds keys 8 (i/4) + 4 (l/32) + i%4, i = 0..15, of row l%32: the row's softmax is lane-local but for
+//   one exchange with the other half-wave, and i/4 is the 8-key group whose exponents apply.
+//   O^T += V^T P^T (dims x rows): A = V^T pieces by transposing LDS reads (ds_read_b64_tr_b16), B = the
+//   lane's own weights split into pieces, so P is never moved between lanes.
+// The softmax weight of a key carries its V exponent, p' = 2^(s + ev - m + 7), so that p' V 2^-ev are
+// the terms of O; the running reference m is an integer, raised only when the maximum passes it by 8
+// (p' <= 2^15), so O is rescaled a few times per row, and s + (ev - m + 7) is one fma of the MFMA's sum.
+//
+// Measured (MI355X), this kernel against the fp32 MFMA one it replaces: a 2048-token prompt, 32/8 heads
+// x 128, 376.7 -> 187.3 us; 333 tokens over 2777 keys, 32/8 heads x 64, F16, 139.4 -> 60.4 us; error
+// against 64 bits 9.2e-7 -> 5.8e-7 and 8.8e-7 -> 4.6e-7 (relative 2-norm).
+#include "dcq_common.h"
+#include "dcq_kernels.h"
+#include "dcq_attn.h"
+
+namespace dcq {
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+
+constexpr int kBlk = 32;        // keys per block
+constexpr int kRows = 128;      // query rows per workgroup
+constexpr float kPOff = 7.0f;   // weights up to 2^7 at their row's reference, 2^15 before it is raised
+
+template <int HD>
+struct __align__(16) PromptSmem {
+    // pitches: K rows are read 16 bytes per lane down a column of 32 rows (4 banks apart); V rows four
+    // at a time, 64 bytes each (16 banks apart)
+    static constexpr int KP = HD + 8, VP = HD + 32;
+    _Float16 k[2][2][kBlk][KP];  // [buffer][piece][key][dim]
+    _Float16 v[2][2][kBlk][VP];
+    float ks[2][4], ev[2][4], vi[2][4];  // per 8 keys: 2^ek, ev, 2^-ev
+};
+
+// The exponent field that normalises magnitudes up to m: m * pow2(268 - E) is in [2^14, 2^15).
+__device__ __forceinline__ int norm_exp(float m) {
+    return max((int)(__float_as_uint(m) >> 23), 30);  // below 2^-97 (zeros too): the floor's exponent
+}
+__device__ __forceinline__ float pow2_bits(int e) { return __uint_as_float((uint32_t)e << 23); }
+
+// four consecutive fp32 values (already scaled) -> the f16 pieces
+__device__ __forceinline__ void split4(const float x0, const float x1, const float x2, const float x3, f16x4& h,
+                                       f16x4& l) {
+    const f16x2 h0 = __builtin_convertvector((f32x2){x0, x1}, f16x2);
+    const f16x2 h1 = __builtin_convertvector((f32x2){x2, x3}, f16x2);
+    const f16x2 l0 = __builtin_convertvector((f32x2){x0 - (float)h0[0], x1 - (float)h0[1]}, f16x2);
+    const f16x2 l1 = __builtin_convertvector((f32x2){x2 - (float)h1[0], x3 - (float)h1[1]}, f16x2);
+    h = __builtin_shufflevector(h0, h1, 0, 1, 2, 3);
+    l = __builtin_shufflevector(l0, l1, 0, 1, 2, 3);
+}
+
+// Transposing LDS read, per 16 lanes: lane j gives the address of elements 4 (j % 4) .. + 3 of row j / 4
+// of a 4 x 16 matrix and receives column j.
+__device__ __forceinline__ f16x4 lds_transposed(const _Float16* src) {
+    typedef short i16x4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) i16x4 LdsI16x4;
+    return __builtin_bit_cast(f16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4*)src));
+}
+
+// One staging thread's E elements of a K (V) row, as loaded: fp32 words of a current row, or the
+// slot's words (Q8_0: E / 4 words of quants and the block's scale; F16: E / 2 words).
+template <int E>
+struct RawRow {
+    uint32_t w[E];
+    uint32_t d;
+};
+
+template <int CT, int E>
+__device__ __forceinline__ void load_raw_slot(const uint8_t* head, int e0, RawRow<E>& r) {
+    if constexpr (CT == kTypeQ8_0) {
+        const uint8_t* b = head + (e0 / 32) * 34;
+        r.d = ldu16(b);
+        __builtin_memcpy(r.w, b + 2 + e0 % 32, E);  // 2-byte aligned
+    } else {
+        constexpr int B = CT == kTypeF16 ? 2 : 4;
+#pragma unroll
+        for (int j = 0; j < B * E / 16; ++j) {
+            const uint4 t = ld16(head + B * e0 + 16 * j);
+            r.w[4 * j] = t.x, r.w[4 * j + 1] = t.y, r.w[4 * j + 2] = t.z, r.w[4 * j + 3] = t.w;
+        }
+    }
+}
+
+template <int CT, int E>
+__device__ __forceinline__ void decode_raw(const RawRow<E>& r, bool hist, float (&x)[E]) {
+    if (CT != kTypeF32 && hist) {
+        if constexpr (CT == kTypeQ8_0) {
+            const float d = half_bits_to_float(r.d);
+#pragma unroll
+            for (int j = 0; j < E; ++j) x[j] = d * (float)(int32_t)__builtin_amdgcn_sbfe(r.w[j / 4], 8 * (j % 4), 8);
+        } else {
+#pragma unroll
+            for (int j = 0; j < E; ++j) x[j] = half_bits_to_float(j % 2 ? r.w[j / 2] >> 16 : r.w[j / 2] & 0xFFFF);
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < E; ++j) x[j] = __uint_as_float(r.w[j]);
+    }
+}
+
+// the largest magnitude of the wave's 64 x E elements
+template <int E>
+__device__ __forceinline__ float wave_amax(const float (&x)[E]) {
+    float m = 0.0f;
+#pragma unroll
+    for (int j = 0; j < E; ++j) m = fmaxf(m, fabsf(x[j]));
+    int b = (int)__float_as_uint(m);  // non-negative: ordered as integers
+    b = max(b, __builtin_amdgcn_update_dpp(b, b, 0xB1, 0xF, 0xF, false));   // quad_perm [1,0,3,2]
+    b = max(b, __builtin_amdgcn_update_dpp(b, b, 0x4E, 0xF, 0xF, false));   // quad_perm [2,3,0,1]
+    b = max(b, __builtin_amdgcn_update_dpp(b, b, 0x141, 0xF, 0xF, false));  // row_half_mirror
+    b = max(b, __builtin_amdgcn_update_dpp(b, b, 0x140, 0xF, 0xF, false));  // row_mirror
+    const int s = max(max(__builtin_amdgcn_readlane(b, 0), __builtin_amdgcn_readlane(b, 16)),
+                      max(__builtin_amdgcn_readlane(b, 32), __builtin_amdgcn_readlane(b, 48)));
+    return __uint_as_float((uint32_t)s);
+}
+
+template <int CT, int HD>
+__global__ void __launch_bounds__(256, HD >= 256 ? 1 : 2) attn_prompt_kernel(AttnArgs a) {
+    constexpr int E = HD / 8;    // elements per staging thread
+    constexpr int KS = HD / 16;  // k-steps of the score product
+    constexpr int NT = HD / 32;  // 32-dim tiles of the output
+    using Smem = PromptSmem<HD>;
+    __shared__ Smem sm;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int p = lane >> 5, c32 = lane & 31;
+    const int rep = a.n_head / a.n_head_kv;
+    const int n_rows = a.n_tokens * rep;
+    const int n_qt = (n_rows + kRows - 1) / kRows;
+    const int id = blockIdx.x;
+    const int h_kv = id % a.n_head_kv;
+    const int split = (id / a.n_head_kv) % a.splits;
+    // query tiles see more key blocks the later their tokens: the first half of the launch order takes
+    // the largest tiles, descending, the second half the smallest, ascending, so that the two workgroups
+    // a CU receives (one from each half, in dispatch order) carry about the same keys together
+    const int rank = id / a.n_head_kv / a.splits, half = (n_qt + 1) / 2;
+    const int qt = rank < half ? n_qt - 1 - rank : rank - half;
+    const int64_t hb = CT == kTypeQ8_0 ? (int64_t)(HD / 32) * 34 : (int64_t)HD * (CT == kTypeF16 ? 2 : 4);
+
+    // ---- the lane's query row: pieces of q * scale * log2(e) at dims 16 s + 8 p .. + 7
+    const int r0 = qt * kRows + 32 * wave;  // the wave's first row
+    const int row = r0 + c32;
+    const bool q_ok = row < n_rows;
+    const int tok = (q_ok ? row : 0) / rep, h = h_kv * rep + (q_ok ? row : 0) % rep;
+    f16x8 qh[KS], ql[KS];
+    float qsc;
+    {
+        const float* qp = a.q + (int64_t)tok * a.q_stride + (int64_t)h * HD + 8 * p;
+        float qv[KS][8], m = 0.0f;
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const float4 t = *reinterpret_cast<const float4*>(qp + 16 * s + 4 * j);
+                qv[s][4 * j] = t.x * a.scale_log2e, qv[s][4 * j + 1] = t.y * a.scale_log2e;
+                qv[s][4 * j + 2] = t.z * a.scale_log2e, qv[s][4 * j + 3] = t.w * a.scale_log2e;
+            }
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) m = fmaxf(m, fabsf(qv[s][j]));
+        m = fmaxf(m, __shfl_xor(m, 32, 64));
+        const int e = norm_exp(m);
+        const float f = pow2_bits(268 - e);
+        qsc = pow2_bits(e - 14);
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            f16x4 h0, l0, h1, l1;
+            split4(qv[s][0] * f, qv[s][1] * f, qv[s][2] * f, qv[s][3] * f, h0, l0);
+            split4(qv[s][4] * f, qv[s][5] * f, qv[s][6] * f, qv[s][7] * f, h1, l1);
+            qh[s] = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
+            ql[s] = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
+        }
+    }
+
+    // keys 0 .. n_past + last token are visible to some row of the tile; with key splits this
+    // workgroup takes blocks [split * cps, split * cps + cps) of them (possibly none)
+    const int last_tok = (min((qt + 1) * kRows, n_rows) - 1) / rep;
+    const int nblk = (a.n_past + last_tok + kBlk) / kBlk;
+    const int b_begin = split * a.cps, b_end = min(nblk, b_begin + a.cps);
+    // the wave's rows: keys up to first_vis are visible to all of them, past last_vis to none
+    const int first_vis = a.n_past + min(r0, n_rows - 1) / rep;
+    const int last_vis = r0 < n_rows ? a.n_past + min(r0 + 31, n_rows - 1) / rep : -1;
+
+    // ---- staging: thread -> key tid / 8 of the block, E elements from se0; wave w stages keys 8w..8w+7
+    const int skey = tid >> 3, se0 = E * (tid & 7);
+    RawRow<E> rk, rv;
+    int kind = 0;  // what rk, rv hold: 0 zeros, 1 history words, 2 fp32 words of a current row
+    auto table_of = [&](int bi) {  // the block-table entry of this thread's key in block bi
+        const int lb = (kBlk * bi + skey) / 16;
+        return kBlk * bi + skey < a.n_past && lb < a.n_table ? a.table[lb] : -1;
+    };
+    auto load_block = [&](int bi, int blk) {
+        const int kk = kBlk * bi + skey;
+        kind = 0;
+        if (kk < a.n_past) {
+            if (blk >= 0 && blk < a.n_blocks) {
+                const int64_t off = (((int64_t)blk * a.n_layer + a.layer) * 16 + kk % 16) * a.sb + (int64_t)h_kv * hb;
+                load_raw_slot<CT, E>(a.k_arena + off, se0, rk);
+                load_raw_slot<CT, E>(a.v_arena + off, se0, rv);
+                kind = 1;
+            }
+        } else if (kk < a.n_past + a.n_tokens) {
+            const int64_t off = (int64_t)(kk - a.n_past) * a.kv_stride + (int64_t)h_kv * HD;
+            load_raw_slot<kTypeF32, E>(reinterpret_cast<const uint8_t*>(a.k_cur + off), se0, rk);
+            load_raw_slot<kTypeF32, E>(reinterpret_cast<const uint8_t*>(a.v_cur + off), se0, rv);
+            kind = 2;
+        }
+    };
+    auto store_piece = [&](const float(&x)[E], float f, _Float16* dh, _Float16* dl) {
+#pragma unroll
+        for (int j = 0; j < E; j += 8) {
+            f16x4 h0, l0, h1, l1;
+            split4(x[j] * f, x[j + 1] * f, x[j + 2] * f, x[j + 3] * f, h0, l0);
+            split4(x[j + 4] * f, x[j + 5] * f, x[j + 6] * f, x[j + 7] * f, h1, l1);
+            *reinterpret_cast<f16x8*>(dh + j) = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
+            *reinterpret_cast<f16x8*>(dl + j) = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
+        }
+    };
+    auto commit_block = [&](int buf) {
+        float x[E];
+        if (kind)
+            decode_raw<CT, E>(rk, kind == 1, x);
+        else
+#pragma unroll
+            for (int j = 0; j < E; ++j) x[j] = 0.0f;
+        int e = norm_exp(wave_amax<E>(x));
+        store_piece(x, pow2_bits(268 - e), &sm.k[buf][0][skey][se0], &sm.k[buf][1][skey][se0]);
+        if (lane == 0) sm.ks[buf][wave] = pow2_bits(e - 14);
+        if (kind)
+            decode_raw<CT, E>(rv, kind == 1, x);
+        else
+#pragma unroll
+            for (int j = 0; j < E; ++j) x[j] = 0.0f;
+        e = norm_exp(wave_amax<E>(x));
+        store_piece(x, pow2_bits(268 - e), &sm.v[buf][0][skey][se0], &sm.v[buf][1][skey][se0]);
+        if (lane == 0) {
+            sm.ev[buf][wave] = (float)(e - 141);
+            sm.vi[buf][wave] = pow2_bits(268 - e);
+        }
+    };
+
+    f32x16 o[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[t][v] = 0.0f;
+    float m_run = -INFINITY, l_run = 0.0f;  // l_run: this lane's keys only, until the end
+
+    int blk_next = -1;
+    if (b_begin < b_end) {
+        load_block(b_begin, table_of(b_begin));
+        if (b_begin + 1 < b_end) blk_next = table_of(b_begin + 1);
+        commit_block(0);
+    }
+    __syncthreads();
+    for (int bi = b_begin; bi < b_end; ++bi) {
+        const int kb = kBlk * bi, buf = (bi - b_begin) & 1;
+        const bool more = bi + 1 < b_end;
+        if (more) {
+            load_block(bi + 1, blk_next);
+            if (bi + 2 < b_end) blk_next = table_of(bi + 2);
+        }
+        if (kb <= last_vis) {
+            // ---- S^T = K Q^T
+            f32x16 sc;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) sc[v] = 0.0f;
+            const _Float16* kh = &sm.k[buf][0][c32][8 * p];
+            const _Float16* kl = &sm.k[buf][1][c32][8 * p];
+#pragma unroll
+            for (int s = 0; s < KS; ++s) {
+                const f16x8 fh = *reinterpret_cast<const f16x8*>(kh + 16 * s);
+                const f16x8 fl = *reinterpret_cast<const f16x8*>(kl + 16 * s);
+                sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(fl, qh[s], sc, 0, 0, 0);
+                sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(fh, ql[s], sc, 0, 0, 0);
+                sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(fh, qh[s], sc, 0, 0, 0);
+            }
+
+            // ---- the online softmax of the lane's row over its 16 keys
+            float cj[4], ev[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                cj[j] = sm.ks[buf][j] * qsc;
+                ev[j] = sm.ev[buf][j];
+            }
+            if (kb + kBlk - 1 > first_vis) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    // -inf for either sign of the scale product: cj > 0
+                    if (kb + 8 * (i >> 2) + 4 * p + (i & 3) > a.n_past + tok) sc[i] = -INFINITY;
+                }
+            }
+            float mx = -INFINITY;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) mx = fmaxf(mx, __builtin_fmaf(sc[i], cj[i >> 2], ev[i >> 2]));
+            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            if (__any(mx > m_run + 8.0f)) {
+                const float m_new = mx > m_run + 8.0f ? __builtin_ceilf(mx) : m_run;
+                const float alpha = m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m_run - m_new);
+                l_run *= alpha;
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) o[t][v] *= alpha;
+                m_run = m_new;
+            }
+            const float off = kPOff - (m_run == -INFINITY ? 0.0f : m_run);
+            float pv[16];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float mo = ev[j] + off;
+#pragma unroll
+                for (int i = 4 * j; i < 4 * j + 4; ++i)
+                    pv[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i], cj[j], mo));
+                l_run = __builtin_fmaf((pv[4 * j] + pv[4 * j + 1]) + (pv[4 * j + 2] + pv[4 * j + 3]), sm.vi[buf][j],
+                                       l_run);
+            }
+
+            // ---- O^T += V^T P^T: step s takes the lane's weights i = 8s .. 8s + 7, keys 16s + 4p + 0..3
+            // and 16s + 8 + 4p + 0..3
+            const int vrow = 4 * p + ((lane & 15) >> 2), vcol = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                f16x4 h0, l0, h1, l1;
+                split4(pv[8 * s], pv[8 * s + 1], pv[8 * s + 2], pv[8 * s + 3], h0, l0);
+                split4(pv[8 * s + 4], pv[8 * s + 5], pv[8 * s + 6], pv[8 * s + 7], h1, l1);
+                const f16x8 ph = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
+                const f16x8 pl = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    f16x8 f[2];
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        const f16x4 a0 = lds_transposed(&sm.v[buf][u][16 * s + vrow][32 * t + vcol]);
+                        const f16x4 a1 = lds_transposed(&sm.v[buf][u][16 * s + 8 + vrow][32 * t + vcol]);
+                        f[u] = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
+                    }
+                    o[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[1], ph, o[t], 0, 0, 0);
+                    o[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[0], pl, o[t], 0, 0, 0);
+                    o[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[0], ph, o[t], 0, 0, 0);
+                }
+            }
+        }
+        if (more) commit_block(buf ^ 1);
+        __syncthreads();
+    }
+    l_run += __shfl_xor(l_run, 32, 64);
+
+    // ---- the lane's query row: dims 32t + 8(v/4) + 4p + v%4 of O^T / l, or with key splits
+    // the unnormalised sums and (m, l) for the combine kernel (m = -inf, l = 0 if no key)
+    if (q_ok) {
+        if (a.splits == 1) {
+            float* orow = a.out + (int64_t)tok * a.out_stride + (int64_t)h * HD;
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) orow[32 * t + 8 * (v >> 2) + 4 * p + (v & 3)] = o[t][v] / l_run;
+        } else {
+            const int64_t wrow = ((int64_t)split * a.n_tokens + tok) * a.n_head + h;
+            float* orow = a.ws_o + wrow * HD;
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    *reinterpret_cast<float4*>(orow + 32 * t + 8 * j + 4 * p) =
+                        make_float4(o[t][4 * j], o[t][4 * j + 1], o[t][4 * j + 2], o[t][4 * j + 3]);
+            if (p == 0) {
+                a.ws_ml[2 * wrow] = m_run;
+                a.ws_ml[2 * wrow + 1] = l_run;
+            }
+        }
+    }
+}
+
+hipError_t launch_attn_prompt(int ct, int hd, const AttnArgs& a, hipStream_t st) {
+    const int64_t rows = (int64_t)a.n_tokens * (a.n_head / a.n_head_kv);
+    const int64_t wgs = (rows + kRows - 1) / kRows * a.n_head_kv * a.splits;
+    if (wgs > INT32_MAX) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)wgs);
+#define DCQ_PROMPT_CASE(C, H)                                                       \
+    if (ct == C && hd == H) {                                                       \
+        hipLaunchKernelGGL((attn_prompt_kernel<C, H>), grid, dim3(256), 0, st, a); \
+    } else
+    DCQ_PROMPT_CASE(kTypeQ8_0, 128)
+    DCQ_PROMPT_CASE(kTypeQ8_0, 64)
+    DCQ_PROMPT_CASE(kTypeQ8_0, 256)
+    DCQ_PROMPT_CASE(kTypeF16, 128)
+    DCQ_PROMPT_CASE(kTypeF16, 64)
+    DCQ_PROMPT_CASE(kTypeF16, 256)
+    DCQ_PROMPT_CASE(kTypeF32, 128)
+    DCQ_PROMPT_CASE(kTypeF32, 64)
+    DCQ_PROMPT_CASE(kTypeF32, 256)
+    return hipErrorNotSupported;
+#undef DCQ_PROMPT_CASE
+    return hipGetLastError();
+}
+
+}  // namespace dcq

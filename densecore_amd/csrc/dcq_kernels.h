@@ -194,6 +194,8 @@ hipError_t launch_kv_gather(int ct, const void* arena, int n_blocks, int n_layer
 // Attention over the arena (head_dim 64/128/256); workspace from attn_workspace_bytes (0 when
 // the keys are not split). hipErrorNotSupported for another head_dim or cache type.
 size_t attn_workspace_bytes(int hd, int n_head, int n_head_kv, int n_tokens, int n_past);
+// the least workspace a call is accepted with (at most attn_workspace_bytes)
+size_t attn_workspace_min_bytes(int hd, int n_head, int n_head_kv, int n_tokens, int n_past);
 hipError_t launch_kv_attention(int ct, const void* k_arena, const void* v_arena, int n_blocks, int n_layer, int layer,
                                int64_t sb, const int32_t* table, int n_table, int n_head, int n_head_kv, int hd,
                                const float* q, int64_t q_stride, const float* k_cur, const float* v_cur,

@@ -206,3 +206,74 @@ def test_kv_decode_steps_write_then_attend(KV, dev):
         KV.write(ct, arena_v, n_layer, layer, table, n_past, vc)
         KV.assert_close_attention(to_host(out).reshape(1, n_head, hd), ref, parts, what=f"decode step {step}")
     assert np.array_equal(to_host(cache.k), arena_k) and np.array_equal(to_host(cache.v), arena_v)
+
+
+PROMPT = [
+    # (cache type, n_tokens, n_past, n_head, n_head_kv, head_dim, K scale, V scale): the prompt kernel's
+    # tiles hold 128 (token, head of the group) rows, 32 a wave, and 32 keys a block
+    (Q8_0, 16, 3, 1, 1, 128, 1, 1),        # the fewest rows it takes; one head; three empty waves
+    (Q8_0, 15, 3, 1, 1, 128, 1, 1),        # one fewer: the VALU kernel
+    (F32, 129, 0, 2, 2, 64, 1, 1),         # one row past a tile, no history
+    (F16, 43, 31, 12, 4, 128, 1, 1),       # groups of 3 (129 rows): tokens straddle waves and tiles
+    (Q8_0, 19, 290, 28, 4, 64, 1, 1),      # groups of 7, the keys split over workgroups
+    (F16, 64, 960, 4, 2, 256, 1, 1),       # head_dim 256, exact blocks and tiles, the fewest keys
+    (Q8_0, 33, 990, 8, 8, 256, 1, 1),      # 33 rows over 1023 keys: the VALU kernel
+    (F32, 9, 1300, 8, 1, 256, 1, 1),       # 72 rows, the keys split
+    (F32, 70, 20, 4, 1, 128, 3e-7, 2e5),   # magnitudes past f16's range on either side
+    (F32, 70, 20, 4, 1, 64, 1e-20, 1e20),
+    (F32, 200, 0, 4, 1, 128, 1, 1e-12),
+]
+
+
+@pytest.mark.parametrize("ct,n,n_past,n_head,n_kv,hd,ks,vs", PROMPT)
+def test_kv_attention_prompt(KV, dev, ct, n, n_past, n_head, n_kv, hd, ks, vs):
+    """The prompt kernel at its edges. Relative 2-norm error against the float64 oracle at most 4e-6:
+    four times what fp32 products and sums measure at these lengths (0.9e-6); one missing f16 piece of
+    any operand costs 2^-12 = 2.4e-4."""
+    n_layer, layer, row = 2, 1, n_kv * hd
+    n_blocks = (n_past + 15) // 16 + 3
+    sb = KV.slot_bytes(ct, row)
+    arena_k = np.zeros(n_blocks * n_layer * 16 * sb, np.uint8)
+    arena_v = np.zeros_like(arena_k)
+    table = make_table(max(n_past, 1), n_blocks, 11 + n)
+    seed = 900 + n + n_past + hd
+    ks, vs = np.float32(ks), np.float32(vs)
+    KV.write(ct, arena_k, n_layer, layer, table, 0, ks * synth.normal(n_past * row, seed).reshape(n_past, row))
+    KV.write(ct, arena_v, n_layer, layer, table, 0, vs * synth.normal(n_past * row, seed + 1).reshape(n_past, row))
+    q = synth.normal(n * n_head * hd, seed + 2, 0.0, 2.0).reshape(n, n_head * hd)
+    k_cur = ks * synth.normal(n * row, seed + 3).reshape(n, row)
+    v_cur = vs * synth.normal(n * row, seed + 4).reshape(n, row)
+    k_cur[n // 2] *= np.float32(8)  # one key of another magnitude among its neighbours
+    v_cur[n // 3] *= np.float32(64)
+    scale = np.float32(1.0 / (np.sqrt(hd) * ks))
+    k_all = KV.gather(ct, arena_k, n_layer, layer, table, n_past, k_cur).reshape(-1, n_kv, hd)
+    v_all = KV.gather(ct, arena_v, n_layer, layer, table, n_past, v_cur).reshape(-1, n_kv, hd)
+    ref, _ = KV.attention(q.reshape(n, n_head, hd), k_all, v_all, n_past, scale)
+
+    cache = dc.PagedKVCache(ct, n_blocks, n_layer, n_kv, hd, device=dev)
+    cache.k.copy_(to_dev(arena_k, dev))
+    cache.v.copy_(to_dev(arena_v, dev))
+    args = (layer, to_dev(table, dev), to_dev(q, dev), to_dev(k_cur, dev), to_dev(v_cur, dev), n_past, float(scale))
+    out = to_host(cache.attention(*args)).astype(np.float64).reshape(ref.shape)
+    assert np.linalg.norm(out - ref) <= 4e-6 * np.linalg.norm(ref)
+
+
+def test_kv_attention_prompt_takes_the_splits_its_workspace_holds(KV, dev):
+    """Groups of 1 head, 96 tokens over 1500 keys: the VALU kernel's plan asked for a smaller workspace
+    than the prompt kernel's splits can use; the call runs with either and agrees to fp32 rounding."""
+    import torch
+    n, n_past, n_head, hd = 96, 1500, 2, 128
+    cache = dc.PagedKVCache(F16, n_past // 16 + 2, 1, n_head, hd, device=dev)
+    rows = [to_dev(synth.normal(m * n_head * hd, 40 + i).reshape(m, -1), dev)
+            for i, m in enumerate((n_past, n_past, n, n, n))]
+    table = torch.arange(n_past // 16 + 1, dtype=torch.int32, device=dev)
+    cache.write("k", 0, table, 0, rows[0])
+    cache.write("v", 0, table, 0, rows[1])
+    need = dc.kv_attention_workspace_size(n_head, n_head, hd, n, n_past)
+    outs = []
+    for nbytes in (need, 4 * need):
+        ws = torch.full((nbytes,), 255, dtype=torch.uint8, device=dev)
+        outs.append(to_host(cache.attention(0, table, *rows[2:], n_past, 0.088, workspace=ws)))
+    assert np.array_equal(outs[0], outs[1])
+    with pytest.raises(dc.DcqError):
+        cache.attention(0, table, *rows[2:], n_past, 0.088, workspace=torch.empty(256, dtype=torch.uint8, device=dev))
