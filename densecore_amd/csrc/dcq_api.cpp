@@ -96,6 +96,7 @@ int knob(Knob k) {
         "DCQ_Q4K_SHAPE",    "DCQ_Q4K_NW",  "DCQ_NO_FUSE",      "DCQ_Q6K_DECODE", "DCQ_Q6K_LDS_OFF",
         "DCQ_Q6K_NO_FUSE",  "DCQ_Q6K_FUSE_NW", "DCQ_Q8_SHAPE", "DCQ_GEMV_GENERIC", "DCQ_GEMV_LG",
         "DCQ_ATTN_NO_MFMA", "DCQ_Q6K_RPW", "DCQ_Q6K_MFMA",     "DCQ_SPLIT_K",    "DCQ_BATCH_MTI",
+        "DCQ_GEMM_MT",      "DCQ_GEMM_KQ",
     };
     static const std::array<int, (int)Knob::kCount> values = [] {
         std::array<int, (int)Knob::kCount> v{};
@@ -404,7 +405,9 @@ int dcq_mul_mat_add(int wtype, const void* W, int64_t N, int64_t K, size_t w_row
     float* T = in_place ? reinterpret_cast<float*>(static_cast<char*>(ws) + act_bytes) : Y;
     const int64_t t_stride = in_place ? N : y_stride;
     // split-K partial sums after the temporary
-    const SplitScratch sc = tail_of(ws, workspace ? workspace_bytes : need, act_bytes + (size_t)M * N * 4);
+    SplitScratch sc = tail_of(ws, workspace ? workspace_bytes : need, act_bytes + (size_t)M * N * 4);
+    AddRows add{R, r_stride, Y, y_stride};
+    sc.add = &add;
     hipError_t e = launch_quantize_planar(vdt, X, (int64_t)(x_stride_bytes / 4), M, K, pb, st);
     bool added = false;
     if (e == hipSuccess && M <= gemv_rows(wtype, N, K, false)) {
@@ -417,7 +420,7 @@ int dcq_mul_mat_add(int wtype, const void* W, int64_t N, int64_t K, size_t w_row
         e = M <= gemv_rows(wtype, N, K, false)
                 ? launch_gemv(wtype, W, (int64_t)w_row_bytes, 0, N, K, pb, M, T, t_stride, nullptr, N, st)
                 : launch_mmq(wtype, W, (int64_t)w_row_bytes, N, K, pb, M, T, t_stride, nullptr, st, sc);
-        if (e == hipSuccess) e = launch_add_rows(Y, y_stride, T, t_stride, R, r_stride, M, N, st);
+        if (e == hipSuccess && !add.done) e = launch_add_rows(Y, y_stride, T, t_stride, R, r_stride, M, N, st);
     }
     if (!workspace) {
         hipError_t e2 = hipFreeAsync(ws, st);
@@ -467,6 +470,18 @@ int dcq_ffn_gate_up(int wtype, const void* Wg, const void* Wu, int64_t N, int64_
     const SplitScratch sc = tail_of(ws, workspace ? workspace_bytes : need, act_bytes + (size_t)M * N * 4);
     hipError_t e = launch_quantize_planar(vdt, X, (int64_t)(x_stride_bytes / 4), M, K, pb, st);
     const bool use_gemv = M <= gemv_rows(wtype, N, K, false);
+    if (e == hipSuccess && !use_gemv && gemm_kq_wins(wtype, M, N, K, true)) {
+        // one kernel: gate and up tiles in one workgroup, their product its store
+        e = launch_gemm_kq(wtype, Wg, Wu, (int64_t)w_row_bytes, N, K, pb, M, Y, y_stride, st);
+        if (e != hipErrorNotSupported) {
+            if (!workspace) {
+                const hipError_t e2 = hipFreeAsync(ws, st);
+                if (e == hipSuccess) e = e2;
+            }
+            return hip_status(e);
+        }
+        e = hipSuccess;
+    }
     if (e == hipSuccess)
         e = use_gemv ? launch_gemv(wtype, Wg, (int64_t)w_row_bytes, 0, N, K, pb, M, Y, y_stride, nullptr, N, st)
                      : launch_mmq(wtype, Wg, (int64_t)w_row_bytes, N, K, pb, M, Y, y_stride, nullptr, st, sc);

@@ -266,7 +266,7 @@ hipError_t launch_batch_q6k(const void* W, int64_t w_row_bytes, int64_t N, int64
     hipLaunchKernelGGL(fn, grid, dim3(64 * kWaves), lds, st, (const uint8_t*)W, w_row_bytes, (int)N, nsb, sp.stps,
                        act.qs, act.d, act.m_ld, (int)M, out, out_stride, block_sums);
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess && sp.splits > 1) e = launch_sum_splits(sc.p, sp.splits, M, N, Y, y_stride, st);
+    if (e == hipSuccess && sp.splits > 1) e = launch_sum_splits(sc, sp.splits, M, N, Y, y_stride, st);
     return e;
 }
 

@@ -320,7 +320,7 @@ hipError_t launch_batch_q8_0(int fmt, const void* W, int64_t w_row_bytes, int64_
     hipLaunchKernelGGL(fn, grid, dim3(64 * kWaves), lds, st, (const uint8_t*)W, w_row_bytes, (int)N, nch, sp.stps,
                        act.qs, act.d, act.m_ld, (int)M, out, out_stride, block_sums);
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess && sp.splits > 1) e = launch_sum_splits(sc.p, sp.splits, M, N, Y, y_stride, st);
+    if (e == hipSuccess && sp.splits > 1) e = launch_sum_splits(sc, sp.splits, M, N, Y, y_stride, st);
     return e;
 }
 

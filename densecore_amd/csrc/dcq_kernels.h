@@ -59,10 +59,12 @@ enum class Knob {
     Q6KMfma,      // DCQ_Q6K_MFMA: 0 keeps tall Q6_K matrices on the lane-per-superblock kernels
     SplitK,       // DCQ_SPLIT_K: force the K splits of the MFMA prefill kernels (-1: rule, 1: none)
     BatchTile,    // DCQ_BATCH_MTI: force the Q4_K batch kernel's 32-row m-tiles per workgroup (1 or 2)
+    GemmMt,       // DCQ_GEMM_MT: force the K-quant GEMM's 32-row m-tiles per workgroup (1, 2, 4; -1: rule)
+    GemmKq,       // DCQ_GEMM_KQ: 0 keeps K-quant products off the GEMM kernel, 1 forces them on it (-1: rule)
     kCount
 };
 // defaults, in Knob order: the launchers' measured rules
-constexpr int kKnobDefault[(int)Knob::kCount] = {-1, 4, 0, 0, 0, 0, -1, -1, 0, -1, 0, -1, 1, -1, -1};
+constexpr int kKnobDefault[(int)Knob::kCount] = {-1, 4, 0, 0, 0, 0, -1, -1, 0, -1, 0, -1, 1, -1, -1, -1, -1};
 #ifdef DCQ_TUNING
 int knob(Knob k);
 #else
@@ -121,10 +123,22 @@ hipError_t launch_decode_fused_q8_0(int fmt, const void* W, int64_t w_row_bytes,
                                     int32_t* block_sums, hipStream_t st, const float* R = nullptr,
                                     int64_t r_stride = 0);
 
+// A residual or bias that a product's last kernel may add on its way out: Y = product + R (row stride
+// r_stride floats, 0: one row), element by element, so R may be Y. done: whether it did; otherwise the
+// product went to the launch's own output and the add is still to do.
+struct AddRows {
+    const float* R;
+    int64_t r_stride;
+    float* Y;
+    int64_t y_stride;
+    bool done = false;
+};
+
 // Room for the partial tiles of a split-K product (fp32 planes of M x N); bytes == 0: no split.
 struct SplitScratch {
     float* p = nullptr;
     size_t bytes = 0;
+    AddRows* add = nullptr;  // optional
 };
 
 // Split-K for the 128 x 128-tile MFMA kernels when their tiles cannot fill the chip: the K stages
@@ -137,8 +151,8 @@ struct SplitPlan {
 // us_per_stage: the estimated time of one stage of one workgroup (the cost model's unit)
 SplitPlan plan_split_k(int64_t tiles, int nstages, int align, int64_t M, int64_t N, const SplitScratch& sc,
                        double us_per_stage = 2.0);
-// Y[m][n] = sum over s (in order) of P[s][m][n], P planes of M x N floats.
-hipError_t launch_sum_splits(const float* P, int splits, int64_t M, int64_t N, float* Y, int64_t y_stride,
+// Y[m][n] = sum over s (in order) of sc.p[s][m][n], planes of M x N floats (plus R, to the add's Y, with sc.add).
+hipError_t launch_sum_splits(const SplitScratch& sc, int splits, int64_t M, int64_t N, float* Y, int64_t y_stride,
                              hipStream_t st);
 
 // Q8_0 / Q4_0 / row-split Q8_0 (fmt) prefill: LDS-staged 128 x 128 int8-MFMA tiles (K % 128 == 0,
@@ -153,10 +167,20 @@ hipError_t launch_prefill_q8_0(int fmt, const void* W, int64_t w_row_bytes, int6
 hipError_t launch_prefill_q6_k(const void* W, int64_t w_row_bytes, int64_t N, int64_t K, const PlanarBuffers& act,
                                int64_t M, float* Y, int64_t y_stride, int32_t* block_sums, hipStream_t st,
                                const SplitScratch& sc = SplitScratch());
-// Q4_K (q5: Q5_K) prefill: the same tiling (K % 256 == 0, w_row_bytes % 16 == 0, m_ld % 128 == 0).
+// Q4_K (q5: Q5_K) prefill with the block sums dumped: the same tiling (K % 256 == 0, w_row_bytes % 16 == 0,
+// m_ld % 128 == 0).
 hipError_t launch_prefill_q4_k(bool q5, const void* W, int64_t w_row_bytes, int64_t N, int64_t K,
                                const PlanarBuffers& act, int64_t M, float* Y, int64_t y_stride, int32_t* block_sums,
                                hipStream_t st, const SplitScratch& sc = SplitScratch());
+
+// Q4_K, Q5_K, Q6_K products of many rows with the weight operands built in registers (K % 256 == 0,
+// m_ld % 128 == 0). W2: the up matrix of a gate/up pair (Y = silu(W x) * (W2 x)), or null. Splits K (plain
+// products) where sc has room, and adds sc.add's rows.
+hipError_t launch_gemm_kq(int wtype, const void* W, const void* W2, int64_t w_row_bytes, int64_t N, int64_t K,
+                          const PlanarBuffers& act, int64_t M, float* Y, int64_t y_stride, hipStream_t st,
+                          const SplitScratch& sc = SplitScratch());
+// Whether launch_gemm_kq is the faster kernel for a product (glu: a gate/up pair); false for other types.
+bool gemm_kq_wins(int wtype, int64_t M, int64_t N, int64_t K, bool glu);
 
 // Q4_K (q5: Q5_K) batched decode (M <= 128): 8-wave workgroups per 32 weight rows x 64 activation
 // rows, K split over the waves (and over workgroups when the rows are few and sc has room);

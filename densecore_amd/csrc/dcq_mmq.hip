@@ -609,6 +609,10 @@ hipError_t launch_mmq(int wtype, const void* W, int64_t w_row_bytes, int64_t N, 
     // 25.5 -> 33.3 us, and at K >= 8192 from 128 rows)
     const bool batch_past_64 =
         M <= 256 && K <= 4096 && ((N + 31) / 32) * ((M + 63) / 64) <= (int64_t)cu_count();
+    if (gemm_kq_wins(wtype, M, N, K, false) && !block_sums) {
+        const hipError_t e = launch_gemm_kq(wtype, W, nullptr, w_row_bytes, N, K, act, M, Y, y_stride, st, sc);
+        if (e != hipErrorNotSupported) return e;
+    }
     // row-split Q8_0: the batched and the 128 x 128-tile kernels (no generic MMQ form)
     if (wtype == kTypeQ8_0_RS) {
         if (M <= 64 || batch_past_64) {
@@ -642,11 +646,8 @@ hipError_t launch_mmq(int wtype, const void* W, int64_t w_row_bytes, int64_t N, 
         const hipError_t e = launch_prefill_q6_k(W, w_row_bytes, N, K, act, M, Y, y_stride, block_sums, st, sc);
         if (e != hipErrorNotSupported) return e;
     }
-    // Q4_K / Q5_K: the batch kernel (64-row m-tiles) up to 256 rows, and up to 512 while the
-    // prefill kernel's 128 x 128 tiles would not give every CU one (steps: 192 x 8192 x 2048 19.9
-    // against 27.8 us on the prefill kernel, 512 x 2048 x 8192 37.5 against 47.4 us, 384 x 8192 x
-    // 2048 36.5 against 39.1 us; but 512 x 8192 x 2048, 256 prefill tiles, 46.3 against 40.6 us, and
-    // from 768 rows the prefill kernel)
+    // Q4_K / Q5_K past the GEMM kernel's rule: the batch kernel (64-row m-tiles) up to 512 rows, the prefill
+    // kernel beyond (it dumps block sums; the products are the GEMM kernel's)
     const bool q4_batch =
         M <= 256 || (M <= 512 && ((M + 127) / 128) * ((N + 127) / 128) < (int64_t)cu_count());
     if ((wtype == kTypeQ4_K || wtype == kTypeQ5_K) && !q4_batch) {

@@ -474,7 +474,7 @@ hipError_t launch_prefill_q8_0(int fmt, const void* W, int64_t w_row_bytes, int6
                        (int)N, (int)K, (int)act.m_ld, (int)w_row_bytes, (const uint8_t*)W, act.qs, act.d, (int)M,
                        sp.stps, out, out_stride, block_sums);
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess && sp.splits > 1) e = launch_sum_splits(sc.p, sp.splits, M, N, Y, y_stride, st);
+    if (e == hipSuccess && sp.splits > 1) e = launch_sum_splits(sc, sp.splits, M, N, Y, y_stride, st);
     return e;
 }
 

@@ -26,7 +26,8 @@
 // becomes the fold at commit, once per weight element per workgroup. LDS rows are 128 bytes of
 // 16-byte slots (one group each), slot XOR (row % 8).
 //
-// Q4_K, vec_dot_q4_K_q8_K's arithmetic, has 8 sub-blocks of 32 with 6-bit scales and mins:
+// Q4_K (for dcq_mul_mat_ex's block sums past the batch kernel's rows only: dcq_gemm_kq.hip serves the
+// products themselves), vec_dot_q4_K_q8_K's arithmetic, has 8 sub-blocks of 32 with 6-bit scales and mins:
 //   Y[m][n] = sum_s dA[m][s] * (d[n][s] * iA - dmin[n][s] * iM)
 //   iA = sum_j sc_j * I_j,  iM = sum_j m_j * S_j   (exact int32; S_j = the activation's sub-block sum)
 // Stages of 128 (half a superblock: 4 sub-blocks) in 128-byte LDS rows; the nibbles are unpacked to one int8
@@ -341,7 +342,7 @@ __global__ void __launch_bounds__(512, 1) prefill_q6_k_kernel(int tiles_n, int t
 // FULL: M and N are multiples of the 128 x 128 tile (no row clamps, unguarded stores).
 // Arguments: the ones the first loads need come first (the first 56 bytes of arguments are
 // preloaded into scalar registers at dispatch).
-template <bool DUMP, bool FULL, bool Q5>
+template <bool FULL, bool Q5>
 __global__ void __launch_bounds__(256, 2) prefill_q4_k_kernel(int tiles_n, int tiles_m, int N, int K, int m_ld,
                                                               int w_row_bytes, const uint8_t* __restrict__ W,
                                                               const int8_t* __restrict__ xqs,
@@ -556,7 +557,7 @@ __global__ void __launch_bounds__(256, 2) prefill_q4_k_kernel(int tiles_n, int t
                         const int iM = (Mh[v] << 6) + Ml[v];  // |iM| <= 8*63*4064 < 2^31
                         const float t = fmaf(-dmj[j].y, (float)iM, dmj[j].x * (float)ai[i][j][v]);
                         acc[i][j][v] = fmaf(da[v], t, acc[i][j][v]);
-                        if (DUMP) {
+                        {
                             const int n = n0 + wn + 32 * j + col;
                             const int m = m0 + wm + 32 * i + 8 * (v >> 2) + 4 * hl + (v & 3);
                             if (m < M && n < N) {
@@ -596,16 +597,14 @@ hipError_t launch_prefill_q4_k(bool q5, const void* W, int64_t w_row_bytes, int6
                                const PlanarBuffers& act, int64_t M, float* Y, int64_t y_stride, int32_t* block_sums,
                                hipStream_t st, const SplitScratch& sc) {
     if (K % 256 || w_row_bytes % 16 || w_row_bytes > INT32_MAX || act.m_ld % kBM || act.m_ld > INT32_MAX ||
-        !act.bs || N > (1 << 30) || M > (1 << 30) || K > (1 << 30))
+        !act.bs || !block_sums || N > (1 << 30) || M > (1 << 30) || K > (1 << 30))
         return hipErrorNotSupported;
     if ((uint64_t)M * (uint64_t)K >= (1ull << 32)) return hipErrorNotSupported;  // 32-bit DMA offsets
     const int tiles_n = (int)((N + kBN - 1) / kBN), tiles_m = (int)((M + kBM - 1) / kBM);
     const size_t lds = 2 * sizeof(StageQ4);
     const bool full = M % kBM == 0 && N % kBN == 0;
-    auto fn = q5 ? (block_sums ? (full ? prefill_q4_k_kernel<true, true, true> : prefill_q4_k_kernel<true, false, true>)
-                               : (full ? prefill_q4_k_kernel<false, true, true> : prefill_q4_k_kernel<false, false, true>))
-                 : (block_sums ? (full ? prefill_q4_k_kernel<true, true, false> : prefill_q4_k_kernel<true, false, false>)
-                               : (full ? prefill_q4_k_kernel<false, true, false> : prefill_q4_k_kernel<false, false, false>));
+    auto fn = q5 ? (full ? prefill_q4_k_kernel<true, true> : prefill_q4_k_kernel<false, true>)
+                 : (full ? prefill_q4_k_kernel<true, false> : prefill_q4_k_kernel<false, false>);
     // split-K when the tiles cannot fill the chip (ranges of whole superblocks: two stages each)
     const SplitPlan sp = plan_split_k((int64_t)tiles_n * tiles_m, (int)(K / kKS), 2, M, N, sc);
     float* out = sp.splits > 1 ? sc.p : Y;
@@ -614,7 +613,7 @@ hipError_t launch_prefill_q4_k(bool q5, const void* W, int64_t w_row_bytes, int6
                        (int)N, (int)K, (int)act.m_ld, (int)w_row_bytes, (const uint8_t*)W, act.qs, act.d,
                        (const int16_t*)act.bs, (int)M, sp.stps, out, out_stride, block_sums);
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess && sp.splits > 1) e = launch_sum_splits(sc.p, sp.splits, M, N, Y, y_stride, st);
+    if (e == hipSuccess && sp.splits > 1) e = launch_sum_splits(sc, sp.splits, M, N, Y, y_stride, st);
     return e;
 }
 
@@ -641,7 +640,7 @@ hipError_t launch_prefill_q6_k(const void* W, int64_t w_row_bytes, int64_t N, in
                        (int)N, (int)K, (int)act.m_ld, (int)w_row_bytes, (const uint8_t*)W, act.qs, act.d, (int)M,
                        sp.stps, out, out_stride, block_sums);
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess && sp.splits > 1) e = launch_sum_splits(sc.p, sp.splits, M, N, Y, y_stride, st);
+    if (e == hipSuccess && sp.splits > 1) e = launch_sum_splits(sc, sp.splits, M, N, Y, y_stride, st);
     return e;
 }
 

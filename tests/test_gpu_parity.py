@@ -745,3 +745,43 @@ def test_batch_small_m(O, dev, wt, M, N, K):
         want = O.block_sums_matrix(wt, K, wq, O.quantize_rows(O.vec_dot_type(wt), x))
         assert np.array_equal(to_host(sums), want)
         O.assert_close(y2, y_ref, l1, RTOL, what=f"batch type {wt} with sums")
+
+
+# The K-quant GEMM with its weight operands built in registers: rows and weight rows around its tiles (32
+# to 128 rows, 128 weight rows, 64 of each matrix of a pair), one superblock and more, every rule that
+# sends a product to it (past 512 rows, tall matrices, few superblocks, an odd number of them for Q6_K).
+GEMM_KQ = [(Q4_K, 513, 97, 256), (Q5_K, 641, 130, 768), (Q4_K, 142, 9217, 256), (Q5_K, 16, 65537, 256),
+           (Q4_K, 5, 32768, 512), (Q6_K, 40, 70, 768), (Q6_K, 129, 16390, 512), (Q6_K, 5, 65537, 256),
+           (Q6_K, 33, 1, 1280), (Q5_K, 33, 25600, 256), (Q4_K, 600, 128, 4096), (Q6_K, 100, 200, 2816)]
+
+
+@pytest.mark.parametrize("wt,M,N,K", GEMM_KQ)
+def test_kquant_gemm(O, dev, wt, M, N, K):
+    """Every output against the oracle: random scale bytes reach the largest folded weights, and rows of one
+    value the largest superblock sums of either sign. With the full workspace (split K where it pays)
+    and the activation-only one, repeated and through dcq_mul_mat_q as test_split_k_parity does."""
+    test_split_k_parity(O, dev, wt, M, N, K)
+    rng = np.random.default_rng(N + K)
+    wq = _random_blocks(wt, N, K, rng)
+    x = synth.normal(M * K, 17).reshape(M, K)
+    x[0] = 3.0
+    x[M - 1] = -3.0
+    y = to_host(dc.mul_mat(wt, to_dev(wq, dev), N, K, to_dev(x, dev)))
+    y_ref, l1 = O.mul_mat(wt, wq, x)
+    # fp32 rounding alone: a few units in the last place of the terms' magnitude per superblock added
+    O.assert_close(y, y_ref, l1, 2.0 ** -22 * (4 + K // 256), what=f"K-quant GEMM type {wt} M={M} N={N} K={K}")
+
+
+@pytest.mark.parametrize("wt,M,N,K", [(Q4_K, 9, 9217, 256), (Q5_K, 65, 8200, 256), (Q6_K, 33, 8129, 512),
+                                      (Q4_K, 513, 63, 512), (Q6_K, 300, 2050, 768), (Q5_K, 520, 65, 1024)])
+def test_ffn_gate_up_gemm(O, dev, wt, M, N, K):
+    test_ffn_gate_up(O, dev, wt, M, N, K)
+
+
+# The add on its way out: the GEMM kernel's store (no split), the split-K sum of the GEMM, batch and
+# prefill kernels (whole quads and odd rows).
+@pytest.mark.parametrize("mode", ["residual", "in_place", "bias"])
+@pytest.mark.parametrize("wt,M,N,K", [(Q4_K, 520, 130, 512), (Q4_K, 600, 128, 4096), (Q6_K, 40, 97, 2816),
+                                      (Q4_0, 13, 256, 4096), (Q8_0, 100, 97, 4096), (Q6_K, 200, 384, 4096)])
+def test_mul_mat_add_on_the_way_out(O, dev, wt, M, N, K, mode):
+    test_mul_mat_add(O, dev, wt, M, N, K, mode)
