@@ -26,6 +26,10 @@ KV_BLOCK_SIZE = 16
 
 PATH_AUTO, PATH_GEMV, PATH_MMQ = 0, 1, 2
 
+# (elements, bytes) of a block of each type, as dcq_block_size and dcq_type_size give them
+_BLOCKS = {0: (1, 4), 1: (1, 2), 2: (32, 18), 8: (32, 34), 12: (256, 144), 13: (256, 176), 14: (256, 210), 15: (256, 292),
+           108: (32, 34)}
+
 _lib = None
 
 
@@ -139,22 +143,57 @@ def mul_mat_workspace_size(wt, m, k):
     return int(lib().dcq_mul_mat_workspace_size(wt, m, k))
 
 
+# The binding's own share of a call is what a decode step waits for beside its launch, so the checks
+# below take one fast path of plain attribute reads and leave every message to the slow one, tensors
+# pass as integer addresses, and nothing calls into the library that is not the call itself
+# (dcq_mul_mat with preallocated tensors: 10.2 -> 6.4 us a call, 3.5 of them the library's and HIP's).
+_torch = _raw_stream = _F32 = _U8 = None
+
+
+def _t():
+    """torch, imported at first use (the metadata calls work without it)."""
+    global _torch, _raw_stream, _F32, _U8
+    if _torch is None:
+        import torch
+        get_stream, get_device = (getattr(torch._C, n, None) for n in ("_cuda_getCurrentRawStream", "_cuda_getDevice"))
+        if get_stream and get_device:
+            _raw_stream = lambda: get_stream(get_device())  # noqa: E731
+        else:
+            _raw_stream = lambda: torch.cuda.current_stream().cuda_stream  # noqa: E731
+        _F32, _U8, _torch = torch.float32, torch.uint8, torch
+    return _torch
+
+
 def _stream(stream):
+    """`stream`, or torch's current stream on the current device (a tensor argument has initialised the
+    device by then; with none, torch.cuda.current_stream() does)."""
     if stream is not None:
-        return ctypes.c_void_p(stream)
-    import torch
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        return stream
+    torch = _t()
+    return _raw_stream() if torch.cuda.is_initialized() else torch.cuda.current_stream().cuda_stream
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
+
+
+def _nbytes(workspace):
+    return workspace.numel() * workspace.element_size() if workspace is not None else 0
+
+
+def _row_bytes(wt, k, w_row_bytes):
+    """The given row stride, or packed rows (dcq_row_size)."""
+    if w_row_bytes is not None:
+        return w_row_bytes
+    block, size = _BLOCKS.get(wt, (1, 0))
+    return k // block * size if k >= 0 and k % block == 0 else 0
 
 
 def _need(name, t, dtype, ndim=(1, 2), cuda=True):
     """Raise ValueError unless t is a tensor of `dtype` with a dimension count in `ndim`, on a GPU
     (when `cuda`), whose last dimension is contiguous: the ABI takes raw pointers and row strides,
     so anything else would be read as the wrong bytes."""
-    import torch
+    torch = _torch or _t()
     if not isinstance(t, torch.Tensor):
         raise ValueError(f"{name}: expected a torch tensor, got {type(t).__name__}")
     if t.dtype != dtype:
@@ -168,18 +207,26 @@ def _need(name, t, dtype, ndim=(1, 2), cuda=True):
 
 
 def _f32(name, t, ndim=(2,)):
-    import torch
-    _need(name, t, torch.float32, ndim)
+    try:
+        if t.dtype is _F32 and t.is_cuda and t.dim() in ndim and t.stride(-1) == 1:
+            return
+    except (AttributeError, IndexError):
+        pass
+    _need(name, t, _t().float32, ndim)
 
 
 def _u8(name, t, ndim=(1, 2)):
-    import torch
-    _need(name, t, torch.uint8, ndim)
+    try:
+        if t.dtype is _U8 and t.is_cuda and t.dim() in ndim and t.stride(-1) == 1:
+            return
+    except (AttributeError, IndexError):
+        pass
+    _need(name, t, _t().uint8, ndim)
 
 
 def quantize_rows(vdt, x, out=None, stream=None):
     """x: float32 cuda [M, K] -> uint8 cuda [M, row_size(vdt, K)] in ggml block layout."""
-    import torch
+    torch = _torch or _t()
     _f32("x", x)
     m, k = x.shape
     if out is None:
@@ -193,17 +240,17 @@ def quantize_rows(vdt, x, out=None, stream=None):
 def mul_mat_ex(wt, wq, n, k, x, y=None, workspace=None, path=PATH_AUTO, block_sums=None, w_row_bytes=None,
                stream=None):
     """Y[M, N] = W[N, K] (quantized rows, uint8 cuda) x X[M, K]^T (float32 cuda)."""
-    import torch
+    torch = _torch or _t()
     _u8("wq", wq)
     _f32("x", x)
     m = x.shape[0]
     if y is None:
         y = torch.empty((m, n), dtype=torch.float32, device=x.device)
-    wrb = w_row_bytes if w_row_bytes is not None else row_size(wt, k)
+    wrb = _row_bytes(wt, k, w_row_bytes)
     _f32("y", y)
     if block_sums is not None:
         _need("block_sums", block_sums, torch.int32, (1, 2, 3))
-    ws_bytes = workspace.numel() * workspace.element_size() if workspace is not None else 0
+    ws_bytes = _nbytes(workspace)
     _check("dcq_mul_mat_ex", lib().dcq_mul_mat_ex(
         wt, _ptr(wq), n, k, wrb, _ptr(x), m, x.stride(0) * 4, _ptr(y), y.stride(0) * 4, _ptr(workspace), ws_bytes,
         path, _ptr(block_sums), _stream(stream)))
@@ -211,15 +258,15 @@ def mul_mat_ex(wt, wq, n, k, x, y=None, workspace=None, path=PATH_AUTO, block_su
 
 
 def mul_mat(wt, wq, n, k, x, y=None, workspace=None, w_row_bytes=None, stream=None):
-    import torch
+    torch = _torch or _t()
     _u8("wq", wq)
     _f32("x", x)
     m = x.shape[0]
     if y is None:
         y = torch.empty((m, n), dtype=torch.float32, device=x.device)
-    wrb = w_row_bytes if w_row_bytes is not None else row_size(wt, k)
+    wrb = _row_bytes(wt, k, w_row_bytes)
     _f32("y", y)
-    ws_bytes = workspace.numel() * workspace.element_size() if workspace is not None else 0
+    ws_bytes = _nbytes(workspace)
     _check("dcq_mul_mat", lib().dcq_mul_mat(
         wt, _ptr(wq), n, k, wrb, _ptr(x), m, x.stride(0) * 4, _ptr(y), y.stride(0) * 4, _ptr(workspace), ws_bytes,
         _stream(stream)))
@@ -236,7 +283,7 @@ def mul_mat_noalloc(wt, wq, n, k, x, y, w_row_bytes=None, stream=None):
     _f32("x", x)
     _f32("y", y)
     m = x.shape[0]
-    wrb = w_row_bytes if w_row_bytes is not None else row_size(wt, k)
+    wrb = _row_bytes(wt, k, w_row_bytes)
     _check("dcq_mul_mat_noalloc", lib().dcq_mul_mat_noalloc(
         wt, _ptr(wq), n, k, wrb, _ptr(x), m, x.stride(0) * 4, _ptr(y), y.stride(0) * 4, _stream(stream)))
     return y
@@ -249,7 +296,7 @@ def mul_mat_add_workspace_size(wt, m, n, k):
 def mul_mat_add(wt, wq, n, k, x, r, y=None, workspace=None, w_row_bytes=None, stream=None):
     """Y[M, N] = W x + R: a projection and its residual (R [M, N], may be y itself) or bias (R [N],
     broadcast over the rows)."""
-    import torch
+    torch = _torch or _t()
     _u8("wq", wq)
     _f32("x", x)
     _f32("r", r, (1, 2))
@@ -258,8 +305,8 @@ def mul_mat_add(wt, wq, n, k, x, r, y=None, workspace=None, w_row_bytes=None, st
         y = torch.empty((m, n), dtype=torch.float32, device=x.device)
     _f32("y", y)
     r_stride = 0 if r.dim() == 1 else r.stride(0) * 4
-    wrb = w_row_bytes if w_row_bytes is not None else row_size(wt, k)
-    ws_bytes = workspace.numel() * workspace.element_size() if workspace is not None else 0
+    wrb = _row_bytes(wt, k, w_row_bytes)
+    ws_bytes = _nbytes(workspace)
     _check("dcq_mul_mat_add", lib().dcq_mul_mat_add(
         wt, _ptr(wq), n, k, wrb, _ptr(x), m, x.stride(0) * 4, _ptr(r), r_stride, _ptr(y), y.stride(0) * 4,
         _ptr(workspace), ws_bytes, _stream(stream)))
@@ -272,16 +319,16 @@ def ffn_gate_up_workspace_size(wt, m, n, k):
 
 def ffn_gate_up(wt, wg, wu, n, k, x, y=None, workspace=None, w_row_bytes=None, stream=None):
     """Y[M, N] = silu(Wg x) * (Wu x): the SwiGLU gate/up pair with one activation quantization."""
-    import torch
+    torch = _torch or _t()
     _u8("wg", wg)
     _u8("wu", wu)
     _f32("x", x)
     m = x.shape[0]
     if y is None:
         y = torch.empty((m, n), dtype=torch.float32, device=x.device)
-    wrb = w_row_bytes if w_row_bytes is not None else row_size(wt, k)
+    wrb = _row_bytes(wt, k, w_row_bytes)
     _f32("y", y)
-    ws_bytes = workspace.numel() * workspace.element_size() if workspace is not None else 0
+    ws_bytes = _nbytes(workspace)
     _check("dcq_ffn_gate_up", lib().dcq_ffn_gate_up(
         wt, _ptr(wg), _ptr(wu), n, k, wrb, _ptr(x), m, x.stride(0) * 4, _ptr(y), y.stride(0) * 4, _ptr(workspace),
         ws_bytes, _stream(stream)))
@@ -342,7 +389,7 @@ class GGUF:
 
     def load(self, i, dst=None, device="cuda:0", stream=None):
         """The tensor's bytes as a uint8 device tensor (rows packed: [ne[1]*..., row bytes])."""
-        import torch
+        torch = _torch or _t()
         meta = self.info(i)
         if dst is None:
             dst = torch.empty(meta["nbytes"], dtype=torch.uint8, device=device)
@@ -353,12 +400,12 @@ class GGUF:
 
 def dot_rows(wt, wq, xq_row, k, n0, n1, y=None, w_row_bytes=None, stream=None):
     """ComputeDotProductBatch: y[r - n0] = vec_dot(W row r, xq_row), xq_row pre-quantized (ggml layout)."""
-    import torch
+    torch = _torch or _t()
     _u8("wq", wq)
     _u8("xq_row", xq_row)
     if y is None:
         y = torch.empty((max(n1 - n0, 0),), dtype=torch.float32, device=wq.device)
-    wrb = w_row_bytes if w_row_bytes is not None else row_size(wt, k)
+    wrb = _row_bytes(wt, k, w_row_bytes)
     _check("dcq_dot_rows", lib().dcq_dot_rows(wt, _ptr(wq), wrb, _ptr(xq_row), k, _ptr(y), n0, n1,
                                               _stream(stream)))
     return y
@@ -366,7 +413,7 @@ def dot_rows(wt, wq, xq_row, k, n0, n1, y=None, w_row_bytes=None, stream=None):
 
 def quantize_weights(wt, w, out=None, stream=None):
     """w: float32 cuda [N, K] -> uint8 cuda [N, row_size(wt, K)] (ggml_quantize_chunk)."""
-    import torch
+    torch = _torch or _t()
     _f32("w", w)
     if not w.is_contiguous():
         raise ValueError("w: rows must be packed (contiguous)")
@@ -380,12 +427,12 @@ def quantize_weights(wt, w, out=None, stream=None):
 def repack_weights(wt, wq, n, k, out_type, out=None, w_row_bytes=None, stream=None):
     """Load-time repack (dcq_repack_weights): N rows of `wt` (uint8 cuda) -> uint8 cuda [N, row_size(out_type, K)]
     rows of out_type (Q8_0 -> row-split Q8_0)."""
-    import torch
+    torch = _torch or _t()
     _u8("wq", wq)
     if out is None:
         out = torch.empty((n, row_size(out_type, k)), dtype=torch.uint8, device=wq.device)
     _u8("out", out)
-    wrb = w_row_bytes if w_row_bytes is not None else row_size(wt, k)
+    wrb = _row_bytes(wt, k, w_row_bytes)
     orb = out.stride(0) if out.dim() == 2 else row_size(out_type, k)
     _check("dcq_repack_weights", lib().dcq_repack_weights(wt, _ptr(wq), n, k, wrb, out_type, _ptr(out), orb,
                                                           _stream(stream)))
@@ -393,11 +440,11 @@ def repack_weights(wt, wq, n, k, out_type, out=None, w_row_bytes=None, stream=No
 
 
 def dequantize_rows(t, wq, n, k, y=None, w_row_bytes=None, stream=None):
-    import torch
+    torch = _torch or _t()
     _u8("wq", wq)
     if y is None:
         y = torch.empty((n, k), dtype=torch.float32, device=wq.device)
-    wrb = w_row_bytes if w_row_bytes is not None else row_size(t, k)
+    wrb = _row_bytes(t, k, w_row_bytes)
     _check("dcq_dequantize_rows", lib().dcq_dequantize_rows(t, _ptr(wq), n, k, wrb, _ptr(y), _stream(stream)))
     return y
 
@@ -414,12 +461,12 @@ def quantize_src1(wt, x, workspace, stream=None):
 
 def mul_mat_q(wt, wq, n, k, workspace, m, y=None, path=PATH_AUTO, w_row_bytes=None, stream=None):
     """Y[M, N] from W and activations already quantized by quantize_src1 into `workspace`."""
-    import torch
+    torch = _torch or _t()
     _u8("wq", wq)
     _u8("workspace", workspace, (1,))
     if y is None:
         y = torch.empty((m, n), dtype=torch.float32, device=wq.device)
-    wrb = w_row_bytes if w_row_bytes is not None else row_size(wt, k)
+    wrb = _row_bytes(wt, k, w_row_bytes)
     _check("dcq_mul_mat_q", lib().dcq_mul_mat_q(wt, _ptr(wq), n, k, wrb, _ptr(workspace), workspace.numel(), m,
                                                 _ptr(y), y.stride(0) * 4, path, _stream(stream)))
     return y
@@ -437,7 +484,7 @@ class PagedKVCache:
     Block tables are int32 device tensors mapping position // 16 to an arena block."""
 
     def __init__(self, cache_type, n_blocks, n_layer, n_head_kv, head_dim, device="cuda"):
-        import torch
+        torch = _torch or _t()
         self.cache_type, self.n_blocks, self.n_layer = cache_type, n_blocks, n_layer
         self.n_head_kv, self.head_dim = n_head_kv, head_dim
         self.row_elems = n_head_kv * head_dim
@@ -453,7 +500,7 @@ class PagedKVCache:
 
     def write(self, which, layer, table, pos0, rows, stream=None):
         """WriteKSlot / WriteVSlot for rows [N, row_elems] at positions pos0 .. pos0 + N - 1."""
-        import torch
+        torch = _torch or _t()
         _f32("rows", rows, (1, 2))
         _need("table", table, torch.int32, (1,))
         _check("dcq_kv_write", lib().dcq_kv_write(
@@ -463,7 +510,7 @@ class PagedKVCache:
 
     def gather(self, which, layer, table, n_past, cur, out=None, stream=None):
         """[n_past + N, row_elems] fp32: history from the cache, then cur (cb_kv_update_and_gather)."""
-        import torch
+        torch = _torch or _t()
         _f32("cur", cur)
         if table is not None:
             _need("table", table, torch.int32, (1,))
@@ -480,7 +527,7 @@ class PagedKVCache:
     def attention(self, layer, table, q, k_cur, v_cur, n_past, scale, out=None, workspace=None, stream=None):
         """q [N, n_head * head_dim] fp32 -> out [N, n_head * head_dim]: causal attention of the N
         batch tokens (positions n_past ..) over the cached history and their own k_cur / v_cur rows."""
-        import torch
+        torch = _torch or _t()
         if k_cur.stride(0) != v_cur.stride(0):
             raise ValueError(f"k_cur and v_cur must share a row stride (the ABI takes one): "
                              f"{k_cur.stride(0)} != {v_cur.stride(0)}")
@@ -493,10 +540,11 @@ class PagedKVCache:
         if out is None:
             out = torch.empty((n, n_head * self.head_dim), dtype=torch.float32, device=q.device)
         _f32("out", out)
-        need = kv_attention_workspace_size(n_head, self.n_head_kv, self.head_dim, n, n_past)
-        if workspace is None and need:
-            workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
-        ws_bytes = workspace.numel() * workspace.element_size() if workspace is not None else 0
+        if workspace is None:
+            need = kv_attention_workspace_size(n_head, self.n_head_kv, self.head_dim, n, n_past)
+            if need:
+                workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
+        ws_bytes = _nbytes(workspace)
         _check("dcq_kv_attention", lib().dcq_kv_attention(
             self.cache_type, _ptr(self.k), _ptr(self.v), self.n_blocks, self.n_layer, layer, _ptr(table),
             table.numel() if table is not None else 0, n_head, self.n_head_kv, self.head_dim, _ptr(q),
