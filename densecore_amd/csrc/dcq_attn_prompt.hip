@@ -119,12 +119,8 @@ __device__ __forceinline__ void decode_raw(const RawRow<E>& r, bool hist, float 
     }
 }
 
-// the largest magnitude of the wave's 64 x E elements
-template <int E>
-__device__ __forceinline__ float wave_amax(const float (&x)[E]) {
-    float m = 0.0f;
-#pragma unroll
-    for (int j = 0; j < E; ++j) m = fmaxf(m, fabsf(x[j]));
+// the largest of the wave's 64 values m >= 0
+__device__ __forceinline__ float wave_max(float m) {
     int b = (int)__float_as_uint(m);  // non-negative: ordered as integers
     b = max(b, __builtin_amdgcn_update_dpp(b, b, 0xB1, 0xF, 0xF, false));   // quad_perm [1,0,3,2]
     b = max(b, __builtin_amdgcn_update_dpp(b, b, 0x4E, 0xF, 0xF, false));   // quad_perm [2,3,0,1]
@@ -133,6 +129,23 @@ __device__ __forceinline__ float wave_amax(const float (&x)[E]) {
     const int s = max(max(__builtin_amdgcn_readlane(b, 0), __builtin_amdgcn_readlane(b, 16)),
                       max(__builtin_amdgcn_readlane(b, 32), __builtin_amdgcn_readlane(b, 48)));
     return __uint_as_float((uint32_t)s);
+}
+
+// The largest finite magnitude of the wave's 64 x E elements: an infinity (its own terms are infinite
+// or NaN) must not set the exponent of the finite elements beside it, which would flush to zero.
+template <int E>
+__device__ __forceinline__ float wave_amax(const float (&x)[E]) {
+    float m = 0.0f;
+#pragma unroll
+    for (int j = 0; j < E; ++j) m = fmaxf(m, fabsf(x[j]));
+    m = wave_max(m);
+    if (m == INFINITY) {  // uniform
+        m = 0.0f;
+#pragma unroll
+        for (int j = 0; j < E; ++j) m = fmaxf(m, fabsf(x[j]) < INFINITY ? fabsf(x[j]) : 0.0f);
+        m = wave_max(m);
+    }
+    return m;
 }
 
 template <int CT, int HD>

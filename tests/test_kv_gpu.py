@@ -277,3 +277,28 @@ def test_kv_attention_prompt_takes_the_splits_its_workspace_holds(KV, dev):
     assert np.array_equal(outs[0], outs[1])
     with pytest.raises(dc.DcqError):
         cache.attention(0, table, *rows[2:], n_past, 0.088, workspace=torch.empty(256, dtype=torch.uint8, device=dev))
+
+
+@pytest.mark.parametrize("ct", [F32, F16])
+def test_kv_attention_prompt_infinite_elements_leave_their_neighbours(dev, ct):
+    """An infinity in one V element changes that dim alone, and one in a K row only the tokens that see
+    the key: the finite elements staged beside them keep their exponents. Against the call without them,
+    to fp32 rounding (4e-6, as above; an element's exponent may move with its neighbours' maximum)."""
+    n, n_past, hd = 48, 40, 64
+    cache = dc.PagedKVCache(ct, 4, 1, 1, hd, device=dev)
+    rows = [to_dev(synth.normal(m * hd * h, 70 + i).reshape(m, -1), dev)
+            for i, (m, h) in enumerate(((n_past, 1), (n_past, 1), (n, 4), (n, 1), (n, 1)))]
+    k_past, v_past, q, k, v = rows
+    table = to_dev(np.array([2, 0, 1], np.int32), dev)
+    outs = []
+    for inf in (False, True):
+        if inf:
+            v_past[5, 3] = float("inf")
+            k[31, 7] = float("inf")
+        cache.write("k", 0, table, 0, k_past)
+        cache.write("v", 0, table, 0, v_past)
+        outs.append(to_host(cache.attention(0, table, q, k, v, n_past, 0.125)).astype(np.float64).reshape(n, 4, hd))
+    dims = [d for d in range(hd) if d != 3]
+    clean, got = outs[0][:31][..., dims], outs[1][:31][..., dims]
+    assert np.linalg.norm(got - clean) <= 4e-6 * np.linalg.norm(clean)
+    assert not np.isfinite(outs[1][:31, :, 3]).any()
