@@ -15,6 +15,13 @@
 // them (one column of MFMA tiles), and walks the keys its rows see in blocks of 32, double-buffered in
 // LDS. The staging of a block (loads, exponents, split) is shared by the 128 rows; its loads are issued
 // before the previous block's MFMAs and its conversion runs after them.
+//   At head_dim 128 a workgroup is two such groups of 4 waves over the same rows, alternate blocks each, and
+//   fills its CU; the second group's sums are added through LDS at the end. As two workgroups of a CU, a
+//   long tile outlived the short one beside it and ran one wave a SIMD, 2.9 us a block against 4.1 us for two
+//   blocks together. The second group converts its next block before its MFMAs, the first after them: one
+//   group's VALU phase meets the other's MFMAs, though both wait at the same barriers. 2048 tokens, 32/8
+//   heads: 198 us as two workgroups, 167 as two groups, 154 with the second one's order turned; 512 tokens
+//   over 4096 keys 161, 156, 152 (events over 20 calls of two KV writes and the attention).
 //   S^T = K Q^T (keys x rows): A = K pieces (16-byte LDS reads), B = Q pieces (registers). Lane l then
 //   holds keys 8 (i/4) + 4 (l/32) + i%4, i = 0..15, of row l%32: the row's softmax is lane-local but for
 //   one exchange with the other half-wave, and i/4 is the 8-key group whose exponents apply.
@@ -25,8 +32,8 @@
 // (p' <= 2^15), so O is rescaled a few times per row, and s + (ev - m + 7) is one fma of the MFMA's sum.
 //
 // Measured (MI355X), this kernel against the fp32 MFMA one it replaces: a 2048-token prompt, 32/8 heads
-// x 128, 376.7 -> 187.3 us; 333 tokens over 2777 keys, 32/8 heads x 64, F16, 139.4 -> 60.4 us; error
-// against 64 bits 9.2e-7 -> 5.8e-7 and 8.8e-7 -> 4.6e-7 (relative 2-norm).
+// x 128, 377 -> 142 us; 333 tokens over 2777 keys, 32/8 heads x 64, F16, 139 -> 60 us; error against 64
+// bits 9.1e-7 -> 5.4e-7 and 8.9e-7 -> 4.6e-7 (relative 2-norm).
 #include "dcq_common.h"
 #include "dcq_kernels.h"
 #include "dcq_attn.h"
@@ -42,6 +49,11 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 constexpr int kBlk = 32;        // keys per block
 constexpr int kRows = 128;      // query rows per workgroup
 constexpr float kPOff = 7.0f;   // weights up to 2^7 at their row's reference, 2^15 before it is raised
+
+// Wave groups of a workgroup: two at head_dim 128. At 256 one group's blocks fill a CU's LDS, and at 64 a CU
+// holds three workgroups of one group, which two groups each measured slower (333 tokens over 2777 keys 67.9
+// -> 74.3 us, 2048 tokens of 14/2 heads 65.4 -> 88.5).
+constexpr int prompt_groups(int hd) { return hd == 128 ? 2 : 1; }
 
 template <int HD>
 struct __align__(16) PromptSmem {
@@ -149,13 +161,16 @@ __device__ __forceinline__ float wave_amax(const float (&x)[E]) {
 }
 
 template <int CT, int HD>
-__global__ void __launch_bounds__(256, HD >= 256 ? 1 : 2) attn_prompt_kernel(AttnArgs a) {
+__global__ void __launch_bounds__(256 * prompt_groups(HD), HD == 64 ? 2 : 1) attn_prompt_kernel(AttnArgs a) {
+    constexpr int G = prompt_groups(HD);
     constexpr int E = HD / 8;    // elements per staging thread
     constexpr int KS = HD / 16;  // k-steps of the score product
     constexpr int NT = HD / 32;  // 32-dim tiles of the output
     using Smem = PromptSmem<HD>;
-    __shared__ Smem sm;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    __shared__ Smem smem[G];
+    const int grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    Smem& sm = smem[grp];
+    const int tid = threadIdx.x & 255, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int p = lane >> 5, c32 = lane & 31;
     const int rep = a.n_head / a.n_head_kv;
     const int n_rows = a.n_tokens * rep;
@@ -163,11 +178,13 @@ __global__ void __launch_bounds__(256, HD >= 256 ? 1 : 2) attn_prompt_kernel(Att
     const int id = blockIdx.x;
     const int h_kv = id % a.n_head_kv;
     const int split = (id / a.n_head_kv) % a.splits;
-    // query tiles see more key blocks the later their tokens: the first half of the launch order takes
-    // the largest tiles, descending, the second half the smallest, ascending, so that the two workgroups
-    // a CU receives (one from each half, in dispatch order) carry about the same keys together
+    // query tiles see more key blocks the later their tokens: largest first, so that the CUs, which take
+    // workgroups as they finish, end together. At head_dim 64, where all of an unsplit launch is resident at
+    // once, the second half of the order takes the smallest tiles, ascending, so that a CU's workgroups (one
+    // from each half, in dispatch order) carry about the same keys together (with splits largest first: 1500
+    // tokens over 100 keys, 24/8 heads, 85.3 -> 74.3 us; 2048 tokens, 14/2 heads, 73.0 -> 65.4)
     const int rank = id / a.n_head_kv / a.splits, half = (n_qt + 1) / 2;
-    const int qt = rank < half ? n_qt - 1 - rank : rank - half;
+    const int qt = HD == 64 && a.splits == 1 && rank >= half ? rank - half : n_qt - 1 - rank;
     const int64_t hb = CT == kTypeQ8_0 ? (int64_t)(HD / 32) * 34 : (int64_t)HD * (CT == kTypeF16 ? 2 : 4);
 
     // ---- the lane's query row: pieces of q * scale * log2(e) at dims 16 s + 8 p .. + 7
@@ -281,20 +298,27 @@ __global__ void __launch_bounds__(256, HD >= 256 ? 1 : 2) attn_prompt_kernel(Att
     float m_run = -INFINITY, l_run = 0.0f;  // l_run: this lane's keys only, until the end
 
     int blk_next = -1;
-    if (b_begin < b_end) {
-        load_block(b_begin, table_of(b_begin));
-        if (b_begin + 1 < b_end) blk_next = table_of(b_begin + 1);
+    const int b0 = b_begin + grp, lead = G == 2 ? grp : 0;  // lead: the group loads one block further ahead
+    if (b0 < b_end) {
+        load_block(b0, table_of(b0));
+        if (b0 + G < b_end) blk_next = table_of(b0 + G);
         commit_block(0);
+        if (lead && b0 + G < b_end) {
+            load_block(b0 + G, blk_next);
+            if (b0 + 2 * G < b_end) blk_next = table_of(b0 + 2 * G);
+        }
     }
     __syncthreads();
-    for (int bi = b_begin; bi < b_end; ++bi) {
-        const int kb = kBlk * bi, buf = (bi - b_begin) & 1;
-        const bool more = bi + 1 < b_end;
-        if (more) {
-            load_block(bi + 1, blk_next);
-            if (bi + 2 < b_end) blk_next = table_of(bi + 2);
+    for (int b = b_begin; b < b_end; b += G) {  // the same turns for every group: barriers
+        const int bi = b + grp, kb = kBlk * bi, buf = (b - b_begin) / G & 1;
+        const bool more = bi + G < b_end;
+        const int nb = bi + G * (1 + lead);
+        if (lead && more) commit_block(buf ^ 1);
+        if (nb < b_end) {
+            load_block(nb, blk_next);
+            if (nb + G < b_end) blk_next = table_of(nb + G);
         }
-        if (kb <= last_vis) {
+        if (bi < b_end && kb <= last_vis) {
             // ---- S^T = K Q^T
             f32x16 sc;
 #pragma unroll
@@ -375,10 +399,34 @@ __global__ void __launch_bounds__(256, HD >= 256 ? 1 : 2) attn_prompt_kernel(Att
                 }
             }
         }
-        if (more) commit_block(buf ^ 1);
+        if (!lead && more) commit_block(buf ^ 1);
         __syncthreads();
     }
     l_run += __shfl_xor(l_run, 32, 64);
+
+    // ---- the second group's sums through LDS (its blocks are done with: the loop ends on a barrier)
+    if constexpr (G == 2) {
+        static_assert((16 * NT + 2) * 256 * sizeof(float) <= sizeof(smem), "");
+        float* part = reinterpret_cast<float*>(smem) + tid;
+        if (grp == 1) {
+            part[0] = m_run, part[256] = l_run;
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) part[256 * (2 + 16 * t + v)] = o[t][v];
+        }
+        __syncthreads();
+        if (grp == 1) return;
+        const float m1 = part[0], m = fmaxf(m_run, m1);
+        const float c0 = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - m);
+        const float c1 = m1 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m1 - m);
+        m_run = m;
+        l_run = l_run * c0 + part[256] * c1;
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) o[t][v] = o[t][v] * c0 + part[256 * (2 + 16 * t + v)] * c1;
+    }
 
     // ---- the lane's query row: dims 32t + 8(v/4) + 4p + v%4 of O^T / l, or with key splits
     // the unnormalised sums and (m, l) for the combine kernel (m = -inf, l = 0 if no key)
@@ -413,7 +461,7 @@ hipError_t launch_attn_prompt(int ct, int hd, const AttnArgs& a, hipStream_t st)
     const dim3 grid((unsigned)wgs);
 #define DCQ_PROMPT_CASE(C, H)                                                       \
     if (ct == C && hd == H) {                                                       \
-        hipLaunchKernelGGL((attn_prompt_kernel<C, H>), grid, dim3(256), 0, st, a); \
+        hipLaunchKernelGGL((attn_prompt_kernel<C, H>), grid, dim3(256 * prompt_groups(H)), 0, st, a); \
     } else
     DCQ_PROMPT_CASE(kTypeQ8_0, 128)
     DCQ_PROMPT_CASE(kTypeQ8_0, 64)

@@ -882,7 +882,7 @@ static size_t attn_partial_bytes(int splits, int hd, int n_head, int n_tokens) {
     return round_up((int64_t)(rows * hd * 4), 256) + round_up((int64_t)(rows * 2 * 4), 256);
 }
 
-// Key splits of the prompt kernel: about 512 workgroups in flight (two per CU; one at head_dim 256),
+// Key splits of the prompt kernel: about 256 workgroups in flight (one per CU; two at head_dim 64),
 // at least 4 key blocks of 32 per split (the last query tile's count; with at least 8, 16 rows over
 // 4096 keys of 8 KV heads x 128 took 26.6 instead of 17.8 us, 128 rows over 300 23.7 instead of
 // 19.4), and no more than the workspace holds.
@@ -891,7 +891,7 @@ struct PromptPlan {
 };
 static PromptPlan attn_prompt_plan(int hd, int n_head, int n_head_kv, int n_tokens, int n_past, size_t ws_bytes) {
     const int64_t rows = (int64_t)n_tokens * (n_head / n_head_kv);
-    const int64_t base = (rows + 127) / 128 * n_head_kv, wgs = hd >= 256 ? 256 : 512;
+    const int64_t base = (rows + 127) / 128 * n_head_kv, wgs = hd == 64 ? 512 : 256;
     const int nblk = (n_past + n_tokens + 31) / 32;
     int64_t want = (wgs + base - 1) / base;
     if (want > (nblk + 3) / 4) want = (nblk + 3) / 4;

@@ -222,6 +222,9 @@ PROMPT = [
     (F32, 70, 20, 4, 1, 128, 3e-7, 2e5),   # magnitudes past f16's range on either side
     (F32, 70, 20, 4, 1, 64, 1e-20, 1e20),
     (F32, 200, 0, 4, 1, 128, 1, 1e-12),
+    (F16, 40, 24, 4, 1, 128, 1, 1),        # two blocks: one for each wave group
+    (Q8_0, 90, 700, 6, 2, 128, 1, 1),      # key splits with odd numbers of blocks
+    (F32, 700, 0, 3, 1, 64, 1, 1),         # a causal prompt with key splits that early tiles do not reach
 ]
 
 
