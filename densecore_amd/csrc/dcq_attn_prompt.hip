@@ -338,13 +338,15 @@ __global__ void __launch_bounds__(256 * prompt_groups(HD), HD == 64 ? 2 : 1) att
             float cj[4], ev[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                cj[j] = sm.ks[buf][j] * qsc;
+                // finite and above 0 whatever the exponents: a score past either end weighs the same, and
+                // the product of two floors (a row and keys of zeros) must not meet the mask as 0 * -inf
+                cj[j] = __builtin_amdgcn_fmed3f(sm.ks[buf][j] * qsc, 0x1p-126f, 0x1.fffffep127f);
                 ev[j] = sm.ev[buf][j];
             }
             if (kb + kBlk - 1 > first_vis) {
 #pragma unroll
                 for (int i = 0; i < 16; ++i) {
-                    // -inf for either sign of the scale product: cj > 0
+                    // a masked key: -inf times cj > 0
                     if (kb + 8 * (i >> 2) + 4 * p + (i & 3) > a.n_past + tok) sc[i] = -INFINITY;
                 }
             }

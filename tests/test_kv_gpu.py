@@ -305,3 +305,64 @@ def test_kv_attention_prompt_infinite_elements_leave_their_neighbours(dev, ct):
     clean, got = outs[0][:31][..., dims], outs[1][:31][..., dims]
     assert np.linalg.norm(got - clean) <= 4e-6 * np.linalg.norm(clean)
     assert not np.isfinite(outs[1][:31, :, 3]).any()
+
+
+def prompt_case(KV, dev, ct, hd, n_head, n_kv, k_past, v_past, q, k_cur, v_cur, scale, holes=()):
+    """One call over a history written to the cache (with `holes` in its block table): the output
+    [n, n_head, hd] in float64, and the oracle's (ref, (A, B)) for the same rows."""
+    n, n_past, row = q.shape[0], k_past.shape[0], n_kv * hd
+    n_blocks = (n_past + 15) // 16 + 2
+    arena_k = np.zeros(n_blocks * 16 * KV.slot_bytes(ct, row), np.uint8)
+    arena_v = np.zeros_like(arena_k)
+    table = make_table(max(n_past, 1), n_blocks, 5 + n, holes)
+    KV.write(ct, arena_k, 1, 0, table, 0, k_past)
+    KV.write(ct, arena_v, 1, 0, table, 0, v_past)
+    k_all = KV.gather(ct, arena_k, 1, 0, table, n_past, k_cur).reshape(-1, n_kv, hd)
+    v_all = KV.gather(ct, arena_v, 1, 0, table, n_past, v_cur).reshape(-1, n_kv, hd)
+    with np.errstate(invalid="ignore"):
+        ref, parts = KV.attention(q.reshape(n, n_head, hd), k_all, v_all, n_past, np.float32(scale))
+    cache = dc.PagedKVCache(ct, n_blocks, 1, n_kv, hd, device=dev)
+    cache.k.copy_(to_dev(arena_k, dev))
+    cache.v.copy_(to_dev(arena_v, dev))
+    out = cache.attention(0, to_dev(table, dev), to_dev(q, dev), to_dev(k_cur, dev), to_dev(v_cur, dev), n_past,
+                          float(scale))
+    return to_host(out).astype(np.float64).reshape(ref.shape), ref, parts
+
+
+def prompt_rows(hd, n_head, n_kv, n_past, n, seed):
+    """k_past, v_past, q, k_cur, v_cur of normal values."""
+    return [synth.normal(m * h * hd, seed + i, 0.0, std).reshape(m, h * hd)
+            for i, (m, h, std) in enumerate(((n_past, n_kv, 1.0), (n_past, n_kv, 1.0), (n, n_head, 2.0),
+                                             (n, n_kv, 1.0), (n, n_kv, 1.0)))]
+
+
+def assert_rows(out, ref, parts):
+    """Every row of every head by itself: |out - ref| <= (2e-6 + 2^-22 B) |A| in the 2-norm. A score of
+    magnitude up to B carries a few units of 2^-24 of B and moves its weight by as much; the weighted sums
+    and the operands' two f16 pieces (22 bits) add a few of 2^-23 of A = sum_t p_t |v_t|."""
+    a, b = parts
+    err = np.linalg.norm(out - ref, axis=2)
+    bound = (2e-6 + 2.0 ** -22 * b) * np.linalg.norm(a, axis=2)
+    bad = ~(err <= bound)
+    assert not bad.any(), f"{int(bad.sum())} of {err.size} rows, first {np.argwhere(bad)[0]}, worst {np.nanmax(err / bound):.3g}"
+
+
+@pytest.mark.parametrize("scale", [None, 0.0])
+@pytest.mark.parametrize("ct,n,n_past,n_head,n_kv,hd", [
+    (F32, 33, 0, 4, 1, 64),       # 1 key past a block of 32, 31 padded ones beside it
+    (F16, 56, 0, 4, 2, 128),      # 24: one padded group of 8 keys
+    (Q8_0, 40, 17, 4, 1, 64),     # 25: no padded group
+    (F32, 48, 16, 2, 1, 128),     # 0: no padding
+    (F16, 19, 1021, 4, 1, 128),   # 16, the keys split over workgroups
+    (Q8_0, 20, 1005, 8, 1, 256),  # 1, split
+    (F32, 160, 1200, 16, 8, 256),  # 16, many tiles
+])
+def test_kv_attention_prompt_zero_rows(KV, dev, ct, n, n_past, n_head, n_kv, hd, scale):
+    """Query rows of zeros (and of 1e-9, and a scale of 0) weigh every visible key alike, also beside
+    keys that are padding: zero rows at the end of the batch, hidden from the rows before them."""
+    k_past, v_past, q, k_cur, v_cur = prompt_rows(hd, n_head, n_kv, n_past, n, 300 + n)
+    q[::3] = 0.0
+    q[1::6] *= np.float32(1e-9)
+    q[-5:], k_cur[-5:], v_cur[-5:] = 0.0, 0.0, 0.0
+    scale = 1.0 / np.sqrt(hd) if scale is None else scale
+    assert_rows(*prompt_case(KV, dev, ct, hd, n_head, n_kv, k_past, v_past, q, k_cur, v_cur, scale))
