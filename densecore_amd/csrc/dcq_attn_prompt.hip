@@ -30,6 +30,12 @@
 // The softmax weight of a key carries its V exponent, p' = 2^(s + ev - m + 7), so that p' V 2^-ev are
 // the terms of O; the running reference m is an integer, raised only when the maximum passes it by 8
 // (p' <= 2^15), so O is rescaled a few times per row, and s + (ev - m + 7) is one fma of the MFMA's sum.
+// The sum of weights is that of p' 2^-ev, which holds while the exponents ev of a row's keys are within 80
+// octaves (kEvMin .. kEvMax, keys of zeros at the lower end): a key as probable as the row's best then has
+// p' >= 2^-75. A group beyond them is staged with the exponent kWide, whose sum with any score asks for a new
+// reference; from there on the wave sums the weights against a reference of their own, straight from the
+// scores (one exp2 more per weight), and takes the groups' true exponents. Blocks of ordinary values pay
+// nothing for it: the branch is that of the reference.
 //
 // Measured (MI355X), this kernel against the fp32 MFMA one it replaces: a 2048-token prompt, 32/8 heads
 // x 128, 377 -> 142 us; 333 tokens over 2777 keys, 32/8 heads x 64, F16, 139 -> 60 us; error against 64
@@ -49,6 +55,10 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 constexpr int kBlk = 32;        // keys per block
 constexpr int kRows = 128;      // query rows per workgroup
 constexpr float kPOff = 7.0f;   // weights up to 2^7 at their row's reference, 2^15 before it is raised
+constexpr int kEBias = 141;     // exponent field of a group's largest magnitude - its exponent: 127 + 14
+constexpr int kEvMin = -64, kEvMax = 16;  // values of 2^-50 .. 2^31
+constexpr int kEvFloor = 30 - kEBias;     // norm_exp's smallest
+constexpr float kWide = 0x1p100f;         // in place of an ev outside kEvMin .. kEvMax
 
 // Wave groups of a workgroup: two at head_dim 128. At 256 one group's blocks fill a CU's LDS, and at 64 a CU
 // holds three workgroups of one group, which two groups each measured slower (333 tokens over 2777 keys 67.9
@@ -62,7 +72,8 @@ struct __align__(16) PromptSmem {
     static constexpr int KP = HD + 8, VP = HD + 32;
     _Float16 k[2][2][kBlk][KP];  // [buffer][piece][key][dim]
     _Float16 v[2][2][kBlk][VP];
-    float ks[2][4], ev[2][4], vi[2][4];  // per 8 keys: 2^ek, ev, 2^-ev
+    float ks[2][4], ev[2][4], vi[2][4];  // per 8 keys: 2^ek, ev (or kWide), 2^-ev
+    float ev_true[2][4];                 // ev, zeros at kEvFloor
 };
 
 // The exponent field that normalises magnitudes up to m: m * pow2(268 - E) is in [2^14, 2^15).
@@ -282,11 +293,13 @@ __global__ void __launch_bounds__(256 * prompt_groups(HD), HD == 64 ? 2 : 1) att
         else
 #pragma unroll
             for (int j = 0; j < E; ++j) x[j] = 0.0f;
-        e = norm_exp(wave_amax<E>(x));
+        const float vm = wave_amax<E>(x);
+        e = vm == 0.0f ? kEBias + kEvMin : norm_exp(vm);
         store_piece(x, pow2_bits(268 - e), &sm.v[buf][0][skey][se0], &sm.v[buf][1][skey][se0]);
         if (lane == 0) {
-            sm.ev[buf][wave] = (float)(e - 141);
+            sm.ev[buf][wave] = e < kEBias + kEvMin || e > kEBias + kEvMax ? kWide : (float)(e - kEBias);
             sm.vi[buf][wave] = pow2_bits(268 - e);
+            sm.ev_true[buf][wave] = (float)(vm == 0.0f ? kEvFloor : e - kEBias);
         }
     };
 
@@ -296,6 +309,8 @@ __global__ void __launch_bounds__(256 * prompt_groups(HD), HD == 64 ? 2 : 1) att
 #pragma unroll
         for (int v = 0; v < 16; ++v) o[t][v] = 0.0f;
     float m_run = -INFINITY, l_run = 0.0f;  // l_run: this lane's keys only, until the end
+    bool own_ref = false;  // (uniform) from here on the sum of weights is l_own, in units of 2^m_own
+    float m_own = -INFINITY, l_own = 0.0f;
 
     int blk_next = -1;
     const int b0 = b_begin + grp, lead = G == 2 ? grp : 0;  // lead: the group loads one block further ahead
@@ -354,7 +369,39 @@ __global__ void __launch_bounds__(256 * prompt_groups(HD), HD == 64 ? 2 : 1) att
 #pragma unroll
             for (int i = 0; i < 16; ++i) mx = fmaxf(mx, __builtin_fmaf(sc[i], cj[i >> 2], ev[i >> 2]));
             mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-            if (__any(mx > m_run + 8.0f)) {
+            if (own_ref || __any(mx > m_run + 8.0f)) {
+                const bool wide = __any(fmaxf(fmaxf(ev[0], ev[1]), fmaxf(ev[2], ev[3])) == kWide);
+                if (wide && !own_ref) {
+                    own_ref = true;
+                    m_own = m_run, l_own = l_run;
+                    // while o is zero its reference is still to choose: that of zeros is far above tiny values
+                    float any_o = 0.0f;
+#pragma unroll
+                    for (int t = 0; t < NT; ++t)
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) any_o = fmaxf(any_o, fabsf(o[t][v]));
+                    if (fmaxf(any_o, __shfl_xor(any_o, 32, 64)) == 0.0f) m_run = -INFINITY;
+                }
+                if (own_ref) {
+                    mx = -INFINITY;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) ev[j] = sm.ev_true[buf][j];
+                    float ms = -INFINITY;
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) {
+                        mx = fmaxf(mx, __builtin_fmaf(sc[i], cj[i >> 2], ev[i >> 2]));
+                        ms = fmaxf(ms, sc[i] * cj[i >> 2]);
+                    }
+                    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+                    ms = fmaxf(m_own, __builtin_ceilf(fmaxf(ms, __shfl_xor(ms, 32, 64))));
+                    if (ms != -INFINITY) {
+                        l_own *= __builtin_amdgcn_exp2f(m_own - ms);
+#pragma unroll
+                        for (int i = 0; i < 16; ++i)
+                            l_own += __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i], cj[i >> 2], kPOff - ms));
+                        m_own = ms;
+                    }
+                }
                 const float m_new = mx > m_run + 8.0f ? __builtin_ceilf(mx) : m_run;
                 const float alpha = m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m_run - m_new);
                 l_run *= alpha;
@@ -404,7 +451,19 @@ __global__ void __launch_bounds__(256 * prompt_groups(HD), HD == 64 ? 2 : 1) att
         if (!lead && more) commit_block(buf ^ 1);
         __syncthreads();
     }
+    l_run = own_ref ? l_own : l_run;
     l_run += __shfl_xor(l_run, 32, 64);
+    if (own_ref && l_run > 0.0f && l_run < INFINITY) {
+        // o in the unit of l again: that of l's leading bit, in which o is no larger than a value
+        const int k = __builtin_amdgcn_frexp_expf(l_run);
+        const int eo = (int)__builtin_amdgcn_fmed3f(m_run - m_own - (float)k, -300.0f, 300.0f);
+        l_run = __builtin_amdgcn_ldexpf(l_run, -k);
+        m_run = m_own + (float)k;
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) o[t][v] = __builtin_amdgcn_ldexpf(o[t][v], eo);
+    }
 
     // ---- the second group's sums through LDS (its blocks are done with: the loop ends on a barrier)
     if constexpr (G == 2) {

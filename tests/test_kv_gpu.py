@@ -366,3 +366,38 @@ def test_kv_attention_prompt_zero_rows(KV, dev, ct, n, n_past, n_head, n_kv, hd,
     q[-5:], k_cur[-5:], v_cur[-5:] = 0.0, 0.0, 0.0
     scale = 1.0 / np.sqrt(hd) if scale is None else scale
     assert_rows(*prompt_case(KV, dev, ct, hd, n_head, n_kv, k_past, v_past, q, k_cur, v_cur, scale))
+
+
+@pytest.mark.parametrize("past,cur", [(0.0, 1.0), (0.0, 1e25), (0.0, 1e-30), (1e-30, 1.0), (1.0, 1e30), (1e30, 1e-30),
+                                      (1e-4, 1.0), (1e-36, 1e-36), (1e35, 1e36)])
+@pytest.mark.parametrize("n_past,hd", [(300, 64), (300, 128), (1030, 256)])
+def test_kv_attention_prompt_value_magnitudes(KV, dev, n_past, hd, past, cur):
+    """Values of one magnitude in the history and another in the batch: no key's weight is lost from
+    the sum of weights, whatever its values are beside the others'."""
+    k_past, v_past, q, k_cur, v_cur = prompt_rows(hd, 4, 1, n_past, 40, 400 + hd)
+    v_past, v_cur = v_past * np.float32(past), v_cur * np.float32(cur)
+    assert_rows(*prompt_case(KV, dev, F32, hd, 4, 1, k_past, v_past, q, k_cur, v_cur, 1.0 / np.sqrt(hd)))
+
+
+@pytest.mark.parametrize("n_kv,hd", [(512, 64), (256, 128), (256, 256),  # a workgroup per CU: the keys unsplit
+                                     (2, 64), (2, 128), (2, 256)])       # the keys split
+def test_kv_attention_prompt_missing_history(dev, n_kv, hd):
+    """8200 history positions without a block read as zero rows: score 0, value 0, in the sum of weights."""
+    import torch
+    n, n_past = 33, 8200
+    _, _, q, k, v = prompt_rows(hd, n_kv, n_kv, 0, n, 500)
+    k *= np.float32(3)  # batch keys that outweigh the history for some rows and not for others
+    cache = dc.PagedKVCache(F16, 1, 1, n_kv, hd, device=dev)
+    table = torch.full((n_past // 16 + 1,), -1, dtype=torch.int32, device=dev)
+    scale = np.float32(1.0 / np.sqrt(hd))
+    out = to_host(cache.attention(0, table, to_dev(q, dev), to_dev(k, dev), to_dev(v, dev), n_past, float(scale)))
+    qh, kh, vh = (x.astype(np.float64).reshape(n, n_kv, hd).transpose(1, 0, 2) for x in (q, k, v))
+    s = qh @ kh.transpose(0, 2, 1) * np.float64(scale)
+    sa = np.abs(qh) @ np.abs(kh).transpose(0, 2, 1) * np.float64(scale)
+    hidden = np.triu(np.ones((n, n), bool), 1)
+    s, sa = np.where(hidden, -np.inf, s), np.where(hidden, 0.0, sa)
+    m = np.maximum(s.max(2, keepdims=True), 0.0)
+    p = np.exp(s - m)
+    p /= n_past * np.exp(-m) + p.sum(2, keepdims=True)
+    ref, a = (p @ vh).transpose(1, 0, 2), (p @ np.abs(vh)).transpose(1, 0, 2)
+    assert_rows(out.astype(np.float64).reshape(ref.shape), ref, (a, sa.max(2).T))
