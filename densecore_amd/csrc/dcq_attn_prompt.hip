@@ -7,8 +7,8 @@
 // and a product takes three MFMAs: h h' + h l' + l h'. Two pieces hold 22 bits or more of x, and the
 // dropped l l' is below 2^-22 of the product. The exponents keep the pieces in f16's range for every fp32
 // input: one per query row, and one per 8 keys for K and for V (the wave that stages 8 keys finds
-// their largest magnitude), chosen so that the largest magnitude lands in [2^14, 2^15). Elements down
-// to 2^-16 of it still have a normal l.
+// their largest magnitude), chosen so that the largest magnitude lands in [2^14, 2^15). An element 2^-r of
+// it keeps 22 bits or more for r up to 16, 39 - r beyond.
 //
 // Work split. The query rows of a KV head are the (token, query head of its group) pairs, token-major,
 // so any group size fills the tiles: a workgroup takes 128 consecutive rows, each of its 4 waves 32 of
@@ -32,10 +32,14 @@
 // (p' <= 2^15), so O is rescaled a few times per row, and s + (ev - m + 7) is one fma of the MFMA's sum.
 // The sum of weights is that of p' 2^-ev, which holds while the exponents ev of a row's keys are within 80
 // octaves (kEvMin .. kEvMax, keys of zeros at the lower end): a key as probable as the row's best then has
-// p' >= 2^-75. A group beyond them is staged with the exponent kWide, whose sum with any score asks for a new
-// reference; from there on the wave sums the weights against a reference of their own, straight from the
-// scores (one exp2 more per weight), and takes the groups' true exponents. Blocks of ordinary values pay
-// nothing for it: the branch is that of the reference.
+// p' >= 2^-75.
+// Wide groups. One exponent for 8 keys costs a key bits where another is far larger, be it one that the row
+// does not see. Keys of a group more than kSpread octaves apart get an exponent each, and such a group, or
+// one of values outside kEvMin .. kEvMax, is staged a second time with the exponent kWide, whose sum with
+// any score asks for a new reference. From there on the wave takes each key's exponents and sums the weights
+// against a reference of their own, straight from the scores (one exp2 more per weight). Ordinary groups
+// pay for the test of their spread and a branch that is not taken: 2048 tokens 141 -> 145 us, 333 tokens
+// over 2777 keys 63 -> 64 (a per-key exponent throughout: 151 and 66).
 //
 // Measured (MI355X), this kernel against the fp32 MFMA one it replaces: a 2048-token prompt, 32/8 heads
 // x 128, 377 -> 142 us; 333 tokens over 2777 keys, 32/8 heads x 64, F16, 139 -> 60 us; error against 64
@@ -57,8 +61,10 @@ constexpr int kRows = 128;      // query rows per workgroup
 constexpr float kPOff = 7.0f;   // weights up to 2^7 at their row's reference, 2^15 before it is raised
 constexpr int kEBias = 141;     // exponent field of a group's largest magnitude - its exponent: 127 + 14
 constexpr int kEvMin = -64, kEvMax = 16;  // values of 2^-50 .. 2^31
+constexpr int kEvZero = kEvMin - 1;       // of a group of zeros, kEvFloor where the keys' own exponents count:
 constexpr int kEvFloor = 30 - kEBias;     // norm_exp's smallest
-constexpr float kWide = 0x1p100f;         // in place of an ev outside kEvMin .. kEvMax
+constexpr float kWide = 0x1p100f;         // in place of the ev of a group whose keys' own exponents count
+constexpr int kSpread = 12;               // octaves that the keys of a group may lie apart under one exponent
 
 // Wave groups of a workgroup: two at head_dim 128. At 256 one group's blocks fill a CU's LDS, and at 64 a CU
 // holds three workgroups of one group, which two groups each measured slower (333 tokens over 2777 keys 67.9
@@ -73,12 +79,12 @@ struct __align__(16) PromptSmem {
     _Float16 k[2][2][kBlk][KP];  // [buffer][piece][key][dim]
     _Float16 v[2][2][kBlk][VP];
     float ks[2][4], ev[2][4], vi[2][4];  // per 8 keys: 2^ek, ev (or kWide), 2^-ev
-    float ev_true[2][4];                 // ev, zeros at kEvFloor
+    float ks1[2][kBlk], ev1[2][kBlk];    // per key, only of wide groups: 2^ek, ev
 };
 
 // The exponent field that normalises magnitudes up to m: m * pow2(268 - E) is in [2^14, 2^15).
-__device__ __forceinline__ int norm_exp(float m) {
-    return max((int)(__float_as_uint(m) >> 23), 30);  // below 2^-97 (zeros too): the floor's exponent
+__device__ __forceinline__ int norm_exp(uint32_t bits) {
+    return max((int)(bits >> 23), 30);  // below 2^-97 (zeros too): the floor's exponent
 }
 __device__ __forceinline__ float pow2_bits(int e) { return __uint_as_float((uint32_t)e << 23); }
 
@@ -142,37 +148,49 @@ __device__ __forceinline__ void decode_raw(const RawRow<E>& r, bool hist, float 
     }
 }
 
-// the largest of the wave's 64 values m >= 0
-__device__ __forceinline__ float wave_max(float m) {
+// The largest of a staging thread's values m >= 0 over its key (8 lanes) and over the wave's 8 keys.
+struct KeyMax {
+    uint32_t key, group;  // the bits
+};
+__device__ __forceinline__ KeyMax key_max(float m) {
     int b = (int)__float_as_uint(m);  // non-negative: ordered as integers
     b = max(b, __builtin_amdgcn_update_dpp(b, b, 0xB1, 0xF, 0xF, false));   // quad_perm [1,0,3,2]
     b = max(b, __builtin_amdgcn_update_dpp(b, b, 0x4E, 0xF, 0xF, false));   // quad_perm [2,3,0,1]
     b = max(b, __builtin_amdgcn_update_dpp(b, b, 0x141, 0xF, 0xF, false));  // row_half_mirror
+    const int key = b;
     b = max(b, __builtin_amdgcn_update_dpp(b, b, 0x140, 0xF, 0xF, false));  // row_mirror
     const int s = max(max(__builtin_amdgcn_readlane(b, 0), __builtin_amdgcn_readlane(b, 16)),
                       max(__builtin_amdgcn_readlane(b, 32), __builtin_amdgcn_readlane(b, 48)));
-    return __uint_as_float((uint32_t)s);
+    return {(uint32_t)key, (uint32_t)s};
 }
 
-// The largest finite magnitude of the wave's 64 x E elements: an infinity (its own terms are infinite
-// or NaN) must not set the exponent of the finite elements beside it, which would flush to zero.
+// The largest finite magnitudes: an infinity (its own terms are infinite or NaN) must not set the exponent
+// of the finite elements beside it, which would flush to zero.
 template <int E>
-__device__ __forceinline__ float wave_amax(const float (&x)[E]) {
+__device__ __forceinline__ KeyMax key_amax(const float (&x)[E]) {
     float m = 0.0f;
 #pragma unroll
     for (int j = 0; j < E; ++j) m = fmaxf(m, fabsf(x[j]));
-    m = wave_max(m);
-    if (m == INFINITY) {  // uniform
+    KeyMax r = key_max(m);
+    if (r.group == 0x7F800000u) {  // uniform
         m = 0.0f;
 #pragma unroll
         for (int j = 0; j < E; ++j) m = fmaxf(m, fabsf(x[j]) < INFINITY ? fabsf(x[j]) : 0.0f);
-        m = wave_max(m);
+        r = key_max(m);
     }
-    return m;
+    return r;
+}
+
+// Whether the keys of a group lie too far apart for one exponent (zeros are exact under any): an element
+// keeps 39 - r bits when it is 2^-r of what its exponent was chosen for, so within kSpread octaves a key's
+// largest keep 27 or more.
+__device__ __forceinline__ bool uneven_keys(const KeyMax& m) {
+    const uint32_t least = (uint32_t)max((int)m.group - (kSpread << 23), 1);
+    return __any(m.key - 1u < least - 1u);
 }
 
 template <int CT, int HD>
-__global__ void __launch_bounds__(256 * prompt_groups(HD), HD == 64 ? 2 : 1) attn_prompt_kernel(AttnArgs a) {
+__global__ void __launch_bounds__(256 * prompt_groups(HD), HD == 64 ? 3 : 1) attn_prompt_kernel(AttnArgs a) {
     constexpr int G = prompt_groups(HD);
     constexpr int E = HD / 8;    // elements per staging thread
     constexpr int KS = HD / 16;  // k-steps of the score product
@@ -221,7 +239,7 @@ __global__ void __launch_bounds__(256 * prompt_groups(HD), HD == 64 ? 2 : 1) att
 #pragma unroll
             for (int j = 0; j < 8; ++j) m = fmaxf(m, fabsf(qv[s][j]));
         m = fmaxf(m, __shfl_xor(m, 32, 64));
-        const int e = norm_exp(m);
+        const int e = norm_exp(__float_as_uint(m));
         const float f = pow2_bits(268 - e);
         qsc = pow2_bits(e - 14);
 #pragma unroll
@@ -278,29 +296,46 @@ __global__ void __launch_bounds__(256 * prompt_groups(HD), HD == 64 ? 2 : 1) att
             *reinterpret_cast<f16x8*>(dl + j) = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
         }
     };
+    auto decode = [&](const RawRow<E>& r, float(&x)[E]) {
+        if (kind)
+            decode_raw<CT, E>(r, kind == 1, x);
+        else
+#pragma unroll
+            for (int j = 0; j < E; ++j) x[j] = 0.0f;
+    };
+    // the wave's 8 keys under one exponent each for K and V; true if they are a wide group, for commit_wide
     auto commit_block = [&](int buf) {
         float x[E];
-        if (kind)
-            decode_raw<CT, E>(rk, kind == 1, x);
-        else
-#pragma unroll
-            for (int j = 0; j < E; ++j) x[j] = 0.0f;
-        int e = norm_exp(wave_amax<E>(x));
-        store_piece(x, pow2_bits(268 - e), &sm.k[buf][0][skey][se0], &sm.k[buf][1][skey][se0]);
-        if (lane == 0) sm.ks[buf][wave] = pow2_bits(e - 14);
-        if (kind)
-            decode_raw<CT, E>(rv, kind == 1, x);
-        else
-#pragma unroll
-            for (int j = 0; j < E; ++j) x[j] = 0.0f;
-        const float vm = wave_amax<E>(x);
-        e = vm == 0.0f ? kEBias + kEvMin : norm_exp(vm);
-        store_piece(x, pow2_bits(268 - e), &sm.v[buf][0][skey][se0], &sm.v[buf][1][skey][se0]);
+        decode(rk, x);
+        KeyMax m = key_amax<E>(x);
+        bool wide = uneven_keys(m);
+        const int ek = norm_exp(m.group);
+        store_piece(x, pow2_bits(268 - ek), &sm.k[buf][0][skey][se0], &sm.k[buf][1][skey][se0]);
+        if (lane == 0) sm.ks[buf][wave] = pow2_bits(ek - 14);
+        decode(rv, x);
+        m = key_amax<E>(x);
+        wide |= uneven_keys(m);
+        const int ev = m.group ? norm_exp(m.group) : kEBias + kEvZero;
+        store_piece(x, pow2_bits(268 - ev), &sm.v[buf][0][skey][se0], &sm.v[buf][1][skey][se0]);
         if (lane == 0) {
-            sm.ev[buf][wave] = e < kEBias + kEvMin || e > kEBias + kEvMax ? kWide : (float)(e - kEBias);
-            sm.vi[buf][wave] = pow2_bits(268 - e);
-            sm.ev_true[buf][wave] = (float)(vm == 0.0f ? kEvFloor : e - kEBias);
+            sm.ev[buf][wave] = (float)(ev - kEBias);
+            sm.vi[buf][wave] = pow2_bits(268 - ev);
         }
+        return wide || ev < kEBias + kEvZero || ev > kEBias + kEvMax || (m.group && ev == kEBias + kEvZero);
+    };
+    // the same keys again, each under its own exponents
+    auto commit_wide = [&](int buf, int bi) {
+        load_block(bi, table_of(bi));
+        float x[E];
+        decode(rk, x);
+        const int ek = norm_exp(key_amax<E>(x).key);
+        store_piece(x, pow2_bits(268 - ek), &sm.k[buf][0][skey][se0], &sm.k[buf][1][skey][se0]);
+        decode(rv, x);
+        const int ev = norm_exp(key_amax<E>(x).key);
+        store_piece(x, pow2_bits(268 - ev), &sm.v[buf][0][skey][se0], &sm.v[buf][1][skey][se0]);
+        sm.ks1[buf][skey] = pow2_bits(ek - 14);
+        sm.ev1[buf][skey] = (float)(ev - kEBias);
+        sm.ev[buf][wave] = kWide;
     };
 
     f32x16 o[NT];
@@ -317,7 +352,7 @@ __global__ void __launch_bounds__(256 * prompt_groups(HD), HD == 64 ? 2 : 1) att
     if (b0 < b_end) {
         load_block(b0, table_of(b0));
         if (b0 + G < b_end) blk_next = table_of(b0 + G);
-        commit_block(0);
+        if (__builtin_expect(commit_block(0), 0)) commit_wide(0, b0);
         if (lead && b0 + G < b_end) {
             load_block(b0 + G, blk_next);
             if (b0 + 2 * G < b_end) blk_next = table_of(b0 + 2 * G);
@@ -328,7 +363,7 @@ __global__ void __launch_bounds__(256 * prompt_groups(HD), HD == 64 ? 2 : 1) att
         const int bi = b + grp, kb = kBlk * bi, buf = (b - b_begin) / G & 1;
         const bool more = bi + G < b_end;
         const int nb = bi + G * (1 + lead);
-        if (lead && more) commit_block(buf ^ 1);
+        if (lead && more && __builtin_expect(commit_block(buf ^ 1), 0)) commit_wide(buf ^ 1, bi + G);
         if (nb < b_end) {
             load_block(nb, blk_next);
             if (nb + G < b_end) blk_next = table_of(nb + G);
@@ -370,8 +405,11 @@ __global__ void __launch_bounds__(256 * prompt_groups(HD), HD == 64 ? 2 : 1) att
             for (int i = 0; i < 16; ++i) mx = fmaxf(mx, __builtin_fmaf(sc[i], cj[i >> 2], ev[i >> 2]));
             mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
             if (own_ref || __any(mx > m_run + 8.0f)) {
-                const bool wide = __any(fmaxf(fmaxf(ev[0], ev[1]), fmaxf(ev[2], ev[3])) == kWide);
-                if (wide && !own_ref) {
+                int wide = 0;  // (uniform) bit j: group j is wide
+#pragma unroll
+                for (int j = 0; j < 4; ++j) wide |= ev[j] == kWide ? 1 << j : 0;
+                wide = __builtin_amdgcn_readfirstlane(wide);
+                if (__builtin_expect(wide && !own_ref, 0)) {
                     own_ref = true;
                     m_own = m_run, l_own = l_run;
                     // while o is zero its reference is still to choose: that of zeros is far above tiny values
@@ -382,25 +420,38 @@ __global__ void __launch_bounds__(256 * prompt_groups(HD), HD == 64 ? 2 : 1) att
                         for (int v = 0; v < 16; ++v) any_o = fmaxf(any_o, fabsf(o[t][v]));
                     if (fmaxf(any_o, __shfl_xor(any_o, 32, 64)) == 0.0f) m_run = -INFINITY;
                 }
-                if (own_ref) {
-                    mx = -INFINITY;
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) ev[j] = sm.ev_true[buf][j];
+                if (__builtin_expect(own_ref, 0)) {
+                    // the scores themselves, their sum of weights, then the exponents of the terms of O, which
+                    // the fma below is to leave as they are
+                    const float* ks1 = &sm.ks1[buf][4 * p];
+                    const float* ev1 = &sm.ev1[buf][4 * p];
                     float ms = -INFINITY;
 #pragma unroll
                     for (int i = 0; i < 16; ++i) {
-                        mx = fmaxf(mx, __builtin_fmaf(sc[i], cj[i >> 2], ev[i >> 2]));
-                        ms = fmaxf(ms, sc[i] * cj[i >> 2]);
+                        float c = cj[i >> 2];
+                        if (wide & (1 << (i >> 2)))
+                            c = __builtin_amdgcn_fmed3f(ks1[8 * (i >> 2) + (i & 3)] * qsc, 0x1p-126f, 0x1.fffffep127f);
+                        sc[i] *= c;
+                        ms = fmaxf(ms, sc[i]);
                     }
-                    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
                     ms = fmaxf(m_own, __builtin_ceilf(fmaxf(ms, __shfl_xor(ms, 32, 64))));
                     if (ms != -INFINITY) {
                         l_own *= __builtin_amdgcn_exp2f(m_own - ms);
 #pragma unroll
-                        for (int i = 0; i < 16; ++i)
-                            l_own += __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i], cj[i >> 2], kPOff - ms));
+                        for (int i = 0; i < 16; ++i) l_own += __builtin_amdgcn_exp2f(sc[i] + (kPOff - ms));
                         m_own = ms;
                     }
+                    mx = -INFINITY;
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) {
+                        float e = ev[i >> 2] == kEvZero ? kEvFloor : ev[i >> 2];
+                        if (wide & (1 << (i >> 2))) e = ev1[8 * (i >> 2) + (i & 3)];
+                        sc[i] += e;
+                        mx = fmaxf(mx, sc[i]);
+                    }
+                    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) cj[j] = 1.0f, ev[j] = 0.0f;
                 }
                 const float m_new = mx > m_run + 8.0f ? __builtin_ceilf(mx) : m_run;
                 const float alpha = m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m_run - m_new);
@@ -448,7 +499,7 @@ __global__ void __launch_bounds__(256 * prompt_groups(HD), HD == 64 ? 2 : 1) att
                 }
             }
         }
-        if (!lead && more) commit_block(buf ^ 1);
+        if (!lead && more && __builtin_expect(commit_block(buf ^ 1), 0)) commit_wide(buf ^ 1, bi + G);
         __syncthreads();
     }
     l_run = own_ref ? l_own : l_run;

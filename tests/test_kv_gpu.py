@@ -344,7 +344,8 @@ def assert_rows(out, ref, parts):
     err = np.linalg.norm(out - ref, axis=2)
     bound = (2e-6 + 2.0 ** -22 * b) * np.linalg.norm(a, axis=2)
     bad = ~(err <= bound)
-    assert not bad.any(), f"{int(bad.sum())} of {err.size} rows, first {np.argwhere(bad)[0]}, worst {np.nanmax(err / bound):.3g}"
+    assert not bad.any(), (f"{int(bad.sum())} of {err.size} rows, first {np.argwhere(bad)[0]}, "
+                           f"worst {np.nanmax(err / bound):.3g}")
 
 
 @pytest.mark.parametrize("scale", [None, 0.0])
@@ -401,3 +402,22 @@ def test_kv_attention_prompt_missing_history(dev, n_kv, hd):
     p /= n_past * np.exp(-m) + p.sum(2, keepdims=True)
     ref, a = (p @ vh).transpose(1, 0, 2), (p @ np.abs(vh)).transpose(1, 0, 2)
     assert_rows(out.astype(np.float64).reshape(ref.shape), ref, (a, sa.max(2).T))
+
+
+@pytest.mark.parametrize("bits", [10, 20, 30, 40])
+@pytest.mark.parametrize("n_past,hd", [(41, 64), (300, 128), (1040, 256)])
+def test_kv_attention_prompt_outlier_keys(KV, dev, n_past, hd, bits):
+    """A key 2^bits times its neighbours, hidden from a row (a later token) or of no weight for it, costs
+    the keys staged beside it no bits: each row by itself."""
+    n, n_kv, n_head = 37, 2, 6
+    k_past, v_past, q, k_cur, v_cur = prompt_rows(hd, n_head, n_kv, n_past, n, 600 + bits)
+    big = np.float32(2.0 ** bits)
+    q.reshape(n, n_head, hd)[:, :, 5] = 2.0
+    for k, v, t in ((k_past, v_past, 11), (k_past, v_past, n_past - 2), (k_cur, v_cur, 20)):
+        k.reshape(-1, n_kv, hd)[t, :, 5] = -60.0 * np.sqrt(hd)  # score about -173 in base 2
+        v[t] *= big
+    k_cur[29] *= big   # hidden from the rows before
+    v_cur[33] *= big
+    out, ref, (a, b) = prompt_case(KV, dev, F32, hd, n_head, n_kv, k_past, v_past, q, k_cur, v_cur, 1.0 / np.sqrt(hd))
+    b = np.minimum(b, 64.0)  # the scores that weigh anything; those of the outliers are far below them
+    assert_rows(out[:29], ref[:29], (a[:29], b[:29]))
