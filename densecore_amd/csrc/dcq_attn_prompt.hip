@@ -164,29 +164,30 @@ __device__ __forceinline__ KeyMax key_max(float m) {
     return {(uint32_t)key, (uint32_t)s};
 }
 
-// The largest finite magnitudes: an infinity (its own terms are infinite or NaN) must not set the exponent
-// of the finite elements beside it, which would flush to zero.
 template <int E>
 __device__ __forceinline__ KeyMax key_amax(const float (&x)[E]) {
     float m = 0.0f;
 #pragma unroll
     for (int j = 0; j < E; ++j) m = fmaxf(m, fabsf(x[j]));
-    KeyMax r = key_max(m);
-    if (r.group == 0x7F800000u) {  // uniform
-        m = 0.0f;
+    return key_max(m);
+}
+
+// The same of the finite elements: an infinity (its own terms are infinite or NaN) must not set the exponent
+// of the finite ones beside it, which would flush to zero.
+template <int E>
+__device__ __forceinline__ KeyMax key_amax_finite(const float (&x)[E]) {
+    float m = 0.0f;
 #pragma unroll
-        for (int j = 0; j < E; ++j) m = fmaxf(m, fabsf(x[j]) < INFINITY ? fabsf(x[j]) : 0.0f);
-        r = key_max(m);
-    }
-    return r;
+    for (int j = 0; j < E; ++j) m = fmaxf(m, fabsf(x[j]) < INFINITY ? fabsf(x[j]) : 0.0f);
+    return key_max(m);
 }
 
 // Whether the keys of a group lie too far apart for one exponent (zeros are exact under any): an element
 // keeps 39 - r bits when it is 2^-r of what its exponent was chosen for, so within kSpread octaves a key's
-// largest keep 27 or more.
+// largest keep 27 or more. True also where one holds an infinity.
 __device__ __forceinline__ bool uneven_keys(const KeyMax& m) {
     const uint32_t least = (uint32_t)max((int)m.group - (kSpread << 23), 1);
-    return __any(m.key - 1u < least - 1u);
+    return __any(m.key - 1u < least - 1u) || m.group == 0x7F800000u;
 }
 
 template <int CT, int HD>
@@ -323,16 +324,24 @@ __global__ void __launch_bounds__(256 * prompt_groups(HD), HD == 64 ? 3 : 1) att
         }
         return wide || ev < kEBias + kEvZero || ev > kEBias + kEvMax || (m.group && ev == kEBias + kEvZero);
     };
-    // the same keys again, each under its own exponents
+    // the same keys again, each under its own exponents. An infinity's l would be NaN: its pieces are 0 and
+    // itself, of which only l meets one factor alone (h of the other operand), so that its product is
+    // infinite of the right sign, or NaN beside a zero, as in fp32
+    auto store_wide = [&](const float(&x)[E], int e, _Float16* dh, _Float16* dl) {
+        store_piece(x, pow2_bits(268 - e), dh, dl);
+#pragma unroll
+        for (int j = 0; j < E; ++j)
+            if (fabsf(x[j]) == INFINITY) dh[j] = (_Float16)0.0f, dl[j] = (_Float16)x[j];
+    };
     auto commit_wide = [&](int buf, int bi) {
         load_block(bi, table_of(bi));
         float x[E];
         decode(rk, x);
-        const int ek = norm_exp(key_amax<E>(x).key);
-        store_piece(x, pow2_bits(268 - ek), &sm.k[buf][0][skey][se0], &sm.k[buf][1][skey][se0]);
+        const int ek = norm_exp(key_amax_finite<E>(x).key);
+        store_wide(x, ek, &sm.k[buf][0][skey][se0], &sm.k[buf][1][skey][se0]);
         decode(rv, x);
-        const int ev = norm_exp(key_amax<E>(x).key);
-        store_piece(x, pow2_bits(268 - ev), &sm.v[buf][0][skey][se0], &sm.v[buf][1][skey][se0]);
+        const int ev = norm_exp(key_amax_finite<E>(x).key);
+        store_wide(x, ev, &sm.v[buf][0][skey][se0], &sm.v[buf][1][skey][se0]);
         sm.ks1[buf][skey] = pow2_bits(ek - 14);
         sm.ev1[buf][skey] = (float)(ev - kEBias);
         sm.ev[buf][wave] = kWide;

@@ -421,3 +421,27 @@ def test_kv_attention_prompt_outlier_keys(KV, dev, n_past, hd, bits):
     out, ref, (a, b) = prompt_case(KV, dev, F32, hd, n_head, n_kv, k_past, v_past, q, k_cur, v_cur, 1.0 / np.sqrt(hd))
     b = np.minimum(b, 64.0)  # the scores that weigh anything; those of the outliers are far below them
     assert_rows(out[:29], ref[:29], (a[:29], b[:29]))
+
+
+@pytest.mark.parametrize("ct", [F32, F16])
+@pytest.mark.parametrize("hd,n_past", [(64, 40), (128, 300), (256, 1001)])
+def test_kv_attention_prompt_infinities(KV, dev, ct, hd, n_past):
+    """As in fp32 arithmetic: a score of minus infinity has no weight, one of plus infinity makes its row
+    NaN, and an infinite value makes its dim infinite for the rows that see it, and leaves the others."""
+    n, n_head = 48, 4
+    k_past, v_past, q, k_cur, v_cur = prompt_rows(hd, n_head, 1, n_past, n, 700 + hd)
+    q.reshape(n, n_head, hd)[:, :, 7] = 0.5 + np.abs(q.reshape(n, n_head, hd)[:, :, 7])
+    k_past[9, 7] = -np.inf   # no weight for any row
+    k_cur[12, 7] = -np.inf
+    out, ref, parts = prompt_case(KV, dev, ct, hd, n_head, 1, k_past, v_past, q, k_cur, v_cur, 1.0 / np.sqrt(hd))
+    a, b = parts
+    finite = np.where(np.isfinite(b), b, 64.0)  # B without the infinite products
+    assert_rows(out, ref, (a, finite))
+    v_past[5, 3] = np.inf
+    v_past[6, 4] = -np.inf
+    k_cur[41, 7] = np.inf    # rows from 41 on
+    got, _, _ = prompt_case(KV, dev, ct, hd, n_head, 1, k_past, v_past, q, k_cur, v_cur, 1.0 / np.sqrt(hd))
+    assert np.isnan(got[41:]).all()
+    assert (got[:41, :, 3] == np.inf).all() and (got[:41, :, 4] == -np.inf).all()
+    dims = [d for d in range(hd) if d not in (3, 4)]
+    assert_rows(got[:41][..., dims], ref[:41][..., dims], (a[:41][..., dims], finite[:41]))
