@@ -27,12 +27,12 @@
 //   one exchange with the other half-wave, and i/4 is the 8-key group whose exponents apply.
 //   O^T += V^T P^T (dims x rows): A = V^T pieces by transposing LDS reads (ds_read_b64_tr_b16), B = the
 //   lane's own weights split into pieces, so P is never moved between lanes.
-// The softmax weight of a key carries its V exponent, p' = 2^(s + ev - m + 7), so that p' V 2^-ev are
-// the terms of O; the running reference m is an integer, raised only when the maximum passes it by 8
-// (p' <= 2^15), so O is rescaled a few times per row, and s + (ev - m + 7) is one fma of the MFMA's sum.
+// The softmax weight of a key carries its V exponent, p' = 2^(s + ev - m), so that 2^7 p' V 2^-ev are the
+// terms of O; the running reference m is an integer, raised only when the maximum passes it by 8
+// (2^7 p' <= 2^15), so O is rescaled a few times per row, and s + (ev - m) is one fma of the MFMA's sum.
 // The sum of weights is that of p' 2^-ev, which holds while the exponents ev of a row's keys are within 80
 // octaves (kEvMin .. kEvMax, keys of zeros at the lower end): a key as probable as the row's best then has
-// p' >= 2^-75.
+// p' >= 2^-82.
 // Wide groups. One exponent for 8 keys costs a key bits where another is far larger, be it one that the row
 // does not see. Keys of a group more than kSpread octaves apart get an exponent each, and such a group, or
 // one of values outside kEvMin .. kEvMax, is staged a second time with the exponent kWide, whose sum with
@@ -41,9 +41,19 @@
 // pay for the test of their spread and a branch that is not taken: 2048 tokens 141 -> 145 us, 333 tokens
 // over 2777 keys 63 -> 64 (a per-key exponent throughout: 151 and 66).
 //
+// Roundings. What is left of the error is the sums', and the scores' most of it: a rounding at a score of 8
+// moves its weight by 8 x 2^-25. So a score's small products are added up first, where their roundings are
+// small too, and the 8 or 16 h h' MFMAs of head_dim 128 and 256 in two sums; the exponent of a weight near
+// the reference is near 0 when it is rounded (2^7 is a factor of the pieces, not of p'); and at head_dim 256
+// a block's terms of O are added to it in one rounding. Relative 2-norm error against 64 bits, VALU or fp32
+// MFMA kernel before / this kernel with one chain for each sum / as it is: 2048 tokens, 32/8 heads x 128,
+// Q8_0: 9.2e-7 / 5.4e-7 / 3.5e-7; 4 tokens over 4095 keys 4.7e-7 / 7.5e-7 / 3.8e-7; 333 tokens over 2777 keys
+// x 64, F16: 8.9e-7 / 4.6e-7 / 4.0e-7; x 256, 8 tokens over 8000 keys 4.4e-7 / 1.02e-6 / 4.2e-7, 2048 tokens
+// 3.9e-7 / 7.5e-7 / 3.4e-7. Cost, the same calls: 162 -> 166 us, 24.1 -> 24.6, 72.4 -> 72.6, 59.8 -> 62.6,
+// 402 -> 425 (events over 20 calls of two KV writes and the attention).
+//
 // Measured (MI355X), this kernel against the fp32 MFMA one it replaces: a 2048-token prompt, 32/8 heads
-// x 128, 377 -> 142 us; 333 tokens over 2777 keys, 32/8 heads x 64, F16, 139 -> 60 us; error against 64
-// bits 9.1e-7 -> 5.4e-7 and 8.9e-7 -> 4.6e-7 (relative 2-norm).
+// x 128, 377 -> 148 us; 333 tokens over 2777 keys, 32/8 heads x 64, F16, 139 -> 64 us.
 #include "dcq_common.h"
 #include "dcq_kernels.h"
 #include "dcq_attn.h"
@@ -58,7 +68,7 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kBlk = 32;        // keys per block
 constexpr int kRows = 128;      // query rows per workgroup
-constexpr float kPOff = 7.0f;   // weights up to 2^7 at their row's reference, 2^15 before it is raised
+constexpr float kPScale = 128.0f;  // of the weights' pieces: 2^7 at their row's reference, 2^15 before it is raised
 constexpr int kEBias = 141;     // exponent field of a group's largest magnitude - its exponent: 127 + 14
 constexpr int kEvMin = -64, kEvMax = 16;  // values of 2^-50 .. 2^31
 constexpr int kEvZero = kEvMin - 1;       // of a group of zeros, kEvFloor where the keys' own exponents count:
@@ -196,6 +206,7 @@ __global__ void __launch_bounds__(256 * prompt_groups(HD), HD == 64 ? 3 : 1) att
     constexpr int E = HD / 8;    // elements per staging thread
     constexpr int KS = HD / 16;  // k-steps of the score product
     constexpr int NT = HD / 32;  // 32-dim tiles of the output
+    constexpr int KC = HD == 64 ? 1 : 2;  // sums of a score's h h' products
     using Smem = PromptSmem<HD>;
     __shared__ Smem smem[G];
     const int grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
@@ -378,19 +389,31 @@ __global__ void __launch_bounds__(256 * prompt_groups(HD), HD == 64 ? 3 : 1) att
             if (nb + G < b_end) blk_next = table_of(nb + G);
         }
         if (bi < b_end && kb <= last_vis) {
-            // ---- S^T = K Q^T
+            // ---- S^T = K Q^T: the small products first, then h h' in KC sums of their own
+            const _Float16* kh = &sm.k[buf][0][c32][8 * p];
+            const _Float16* kl = &sm.k[buf][1][c32][8 * p];
             f32x16 sc;
 #pragma unroll
             for (int v = 0; v < 16; ++v) sc[v] = 0.0f;
-            const _Float16* kh = &sm.k[buf][0][c32][8 * p];
-            const _Float16* kl = &sm.k[buf][1][c32][8 * p];
 #pragma unroll
             for (int s = 0; s < KS; ++s) {
                 const f16x8 fh = *reinterpret_cast<const f16x8*>(kh + 16 * s);
                 const f16x8 fl = *reinterpret_cast<const f16x8*>(kl + 16 * s);
                 sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(fl, qh[s], sc, 0, 0, 0);
                 sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(fh, ql[s], sc, 0, 0, 0);
-                sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(fh, qh[s], sc, 0, 0, 0);
+            }
+#pragma unroll
+            for (int c = 0; c < KC; ++c) {
+                f32x16 d;
+#pragma unroll
+                for (int v = 0; v < 16; ++v) d[v] = c ? 0.0f : sc[v];
+#pragma unroll
+                for (int s = c * KS / KC; s < (c + 1) * KS / KC; ++s) {
+                    const f16x8 fh = *reinterpret_cast<const f16x8*>(kh + 16 * s);
+                    d = __builtin_amdgcn_mfma_f32_32x32x16_f16(fh, qh[s], d, 0, 0, 0);
+                }
+#pragma unroll
+                for (int v = 0; v < 16; ++v) sc[v] = c ? sc[v] + d[v] : d[v];
             }
 
             // ---- the online softmax of the lane's row over its 16 keys
@@ -447,7 +470,7 @@ __global__ void __launch_bounds__(256 * prompt_groups(HD), HD == 64 ? 3 : 1) att
                     if (ms != -INFINITY) {
                         l_own *= __builtin_amdgcn_exp2f(m_own - ms);
 #pragma unroll
-                        for (int i = 0; i < 16; ++i) l_own += __builtin_amdgcn_exp2f(sc[i] + (kPOff - ms));
+                        for (int i = 0; i < 16; ++i) l_own += __builtin_amdgcn_exp2f(sc[i] - ms);
                         m_own = ms;
                     }
                     mx = -INFINITY;
@@ -471,7 +494,7 @@ __global__ void __launch_bounds__(256 * prompt_groups(HD), HD == 64 ? 3 : 1) att
                     for (int v = 0; v < 16; ++v) o[t][v] *= alpha;
                 m_run = m_new;
             }
-            const float off = kPOff - (m_run == -INFINITY ? 0.0f : m_run);
+            const float off = m_run == -INFINITY ? 0.0f : -m_run;
             float pv[16];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -484,17 +507,25 @@ __global__ void __launch_bounds__(256 * prompt_groups(HD), HD == 64 ? 3 : 1) att
             }
 
             // ---- O^T += V^T P^T: step s takes the lane's weights i = 8s .. 8s + 7, keys 16s + 4p + 0..3
-            // and 16s + 8 + 4p + 0..3
+            // and 16s + 8 + 4p + 0..3; at head_dim 256 a block's terms are summed on their own first
             const int vrow = 4 * p + ((lane & 15) >> 2), vcol = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+            f16x8 ph[2], pl[2];
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
                 f16x4 h0, l0, h1, l1;
-                split4(pv[8 * s], pv[8 * s + 1], pv[8 * s + 2], pv[8 * s + 3], h0, l0);
-                split4(pv[8 * s + 4], pv[8 * s + 5], pv[8 * s + 6], pv[8 * s + 7], h1, l1);
-                const f16x8 ph = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
-                const f16x8 pl = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
+                const float* w = pv + 8 * s;
+                split4(w[0] * kPScale, w[1] * kPScale, w[2] * kPScale, w[3] * kPScale, h0, l0);
+                split4(w[4] * kPScale, w[5] * kPScale, w[6] * kPScale, w[7] * kPScale, h1, l1);
+                ph[s] = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
+                pl[s] = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
+            }
 #pragma unroll
-                for (int t = 0; t < NT; ++t) {
+            for (int t = 0; t < NT; ++t) {
+                f32x16 d;
+#pragma unroll
+                for (int v = 0; v < 16; ++v) d[v] = HD == 256 ? 0.0f : o[t][v];
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
                     f16x8 f[2];
 #pragma unroll
                     for (int u = 0; u < 2; ++u) {
@@ -502,16 +533,18 @@ __global__ void __launch_bounds__(256 * prompt_groups(HD), HD == 64 ? 3 : 1) att
                         const f16x4 a1 = lds_transposed(&sm.v[buf][u][16 * s + 8 + vrow][32 * t + vcol]);
                         f[u] = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
                     }
-                    o[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[1], ph, o[t], 0, 0, 0);
-                    o[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[0], pl, o[t], 0, 0, 0);
-                    o[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[0], ph, o[t], 0, 0, 0);
+                    d = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[1], ph[s], d, 0, 0, 0);
+                    d = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[0], pl[s], d, 0, 0, 0);
+                    d = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[0], ph[s], d, 0, 0, 0);
                 }
+#pragma unroll
+                for (int v = 0; v < 16; ++v) o[t][v] = HD == 256 ? o[t][v] + d[v] : d[v];
             }
         }
         if (!lead && more && __builtin_expect(commit_block(buf ^ 1), 0)) commit_wide(buf ^ 1, bi + G);
         __syncthreads();
     }
-    l_run = own_ref ? l_own : l_run;
+    l_run = (own_ref ? l_own : l_run) * kPScale;
     l_run += __shfl_xor(l_run, 32, 64);
     if (own_ref && l_run > 0.0f && l_run < INFINITY) {
         // o in the unit of l again: that of l's leading bit, in which o is no larger than a value
