@@ -41,6 +41,12 @@ def test_version_and_status_strings():
 def test_type_traits_match_gguf():
     assert [dc.block_size(t) for t in (0, 1, 2, 8, 12, 13, 14, 15, 3)] == [1, 1, 32, 32, 256, 256, 256, 256, 0]
     assert [dc.type_size(t) for t in (0, 1, 2, 8, 12, 13, 14, 15)] == [4, 2, 18, 34, 144, 176, 210, 292]
+    # the binding's own table, which the calls take packed row strides from
+    types = [t for t in range(128) if dc.block_size(t)]
+    assert dc._lib._BLOCKS == {t: (dc.block_size(t), dc.type_size(t)) for t in types}
+    for t in range(-1, 128):
+        for k in (-256, 0, 32, 256, 1000, 2560):
+            assert dc._lib._row_bytes(t, k, None) == dc.row_size(t, k)
     assert dc.row_size(2, 2560) == 1440
     assert dc.row_size(13, 2560) == 1760
     assert dc.row_size(8, 1024) == 1088

@@ -43,6 +43,8 @@ MUL_MAT = [
     (Q6_K, 1, 1024, 2560),   # fused Q6_K decode
     (Q4_K, 64, 512, 2048),   # quantize + batched MFMA kernel
     (Q8_0, 256, 512, 2048),  # quantize + prefill MFMA kernel
+    (Q4_K, 520, 640, 1024),  # quantize + K-quant GEMM
+    (Q6_K, 40, 128, 2816),   # ... and its split-K sum
 ]
 
 
@@ -58,21 +60,22 @@ def test_mul_mat_graph_replays(dev, wt, M, N, K):
                                       stream=torch.cuda.current_stream().cuda_stream), [y])
 
 
-def test_gate_up_graph_replays(dev):
+@pytest.mark.parametrize("M,N,K", [(1, 9728, 2560), (72, 8192, 512)])  # fused decode; the GEMM of the pair
+def test_gate_up_graph_replays(dev, M, N, K):
     import torch
-    N, K = 9728, 2560
     wg = dc.quantize_weights(Q4_K, torch.from_numpy(synth.normal(N * K, 7, 0.0, 0.02).reshape(N, K)).to(dev))
     wu = dc.quantize_weights(Q4_K, torch.from_numpy(synth.normal(N * K, 8, 0.0, 0.02).reshape(N, K)).to(dev))
-    x = torch.from_numpy(synth.normal(K, 9).reshape(1, K)).to(dev)
-    y = torch.empty((1, N), dtype=torch.float32, device=dev)
-    ws = torch.empty(max(dc.ffn_gate_up_workspace_size(Q4_K, 1, N, K), 256), dtype=torch.uint8, device=dev)
+    x = torch.from_numpy(synth.normal(M * K, 9).reshape(M, K)).to(dev)
+    y = torch.empty((M, N), dtype=torch.float32, device=dev)
+    ws = torch.empty(max(dc.ffn_gate_up_workspace_size(Q4_K, M, N, K), 256), dtype=torch.uint8, device=dev)
     _replays_match(lambda: dc.ffn_gate_up(Q4_K, wg, wu, N, K, x, y=y, workspace=ws,
                                           stream=torch.cuda.current_stream().cuda_stream), [y])
 
 
-@pytest.mark.parametrize("wt,M,N,K", [(Q4_K, 1, 2560, 9728), (Q6_K, 1, 2560, 9728), (Q8_0, 64, 256, 1024)])
+@pytest.mark.parametrize("wt,M,N,K", [(Q4_K, 1, 2560, 9728), (Q6_K, 1, 2560, 9728), (Q8_0, 64, 256, 1024),
+                                      (Q4_K, 520, 128, 4096)])
 def test_mul_mat_add_graph_replays(dev, wt, M, N, K):
-    """Projection + residual in a graph: the fused store epilogue and the add kernel after."""
+    """Projection + residual in a graph: the fused store epilogue, the add kernel after, the add in the split-K sum."""
     import torch
     w = torch.from_numpy(synth.normal(N * K, 14, 0.0, 0.02).reshape(N, K)).to(dev)
     wq = dc.quantize_weights(wt, w)

@@ -332,7 +332,7 @@ def test_untracked_loads_and_lds_loads_are_waited_for(kernel_asm):
     # loads in every staged kernel
     assert totals["dcq_decode_q6.hip"][0] > 0
     for f in ("dcq_prefill.hip", "dcq_prefill_kq.hip", "dcq_batch.hip", "dcq_batch_q8.hip", "dcq_batch_q6.hip",
-              "dcq_decode_q6.hip"):
+              "dcq_decode_q6.hip", "dcq_gemm_kq.hip"):
         assert totals[f][1] > 0, f
 
 

@@ -208,6 +208,47 @@ def test_kv_decode_steps_write_then_attend(KV, dev):
     assert np.array_equal(to_host(cache.k), arena_k) and np.array_equal(to_host(cache.v), arena_v)
 
 
+def prompt_case(KV, dev, ct, hd, n_head, n_kv, k_past, v_past, q, k_cur, v_cur, scale, holes=()):
+    """One call over a history written to the cache (with `holes` in its block table): the output
+    [n, n_head, hd] in float64, and the oracle's (ref, (A, B)) for the same rows."""
+    n, n_past, row = q.shape[0], k_past.shape[0], n_kv * hd
+    n_blocks = (n_past + 15) // 16 + 2
+    arena_k = np.zeros(n_blocks * 16 * KV.slot_bytes(ct, row), np.uint8)
+    arena_v = np.zeros_like(arena_k)
+    table = make_table(max(n_past, 1), n_blocks, 5 + n, holes)
+    KV.write(ct, arena_k, 1, 0, table, 0, k_past)
+    KV.write(ct, arena_v, 1, 0, table, 0, v_past)
+    k_all = KV.gather(ct, arena_k, 1, 0, table, n_past, k_cur).reshape(-1, n_kv, hd)
+    v_all = KV.gather(ct, arena_v, 1, 0, table, n_past, v_cur).reshape(-1, n_kv, hd)
+    with np.errstate(invalid="ignore"):
+        ref, parts = KV.attention(q.reshape(n, n_head, hd), k_all, v_all, n_past, np.float32(scale))
+    cache = dc.PagedKVCache(ct, n_blocks, 1, n_kv, hd, device=dev)
+    cache.k.copy_(to_dev(arena_k, dev))
+    cache.v.copy_(to_dev(arena_v, dev))
+    out = cache.attention(0, to_dev(table, dev), to_dev(q, dev), to_dev(k_cur, dev), to_dev(v_cur, dev), n_past,
+                          float(scale))
+    return to_host(out).astype(np.float64).reshape(ref.shape), ref, parts
+
+
+def prompt_rows(hd, n_head, n_kv, n_past, n, seed):
+    """k_past, v_past, q, k_cur, v_cur of normal values."""
+    return [synth.normal(m * h * hd, seed + i, 0.0, std).reshape(m, h * hd)
+            for i, (m, h, std) in enumerate(((n_past, n_kv, 1.0), (n_past, n_kv, 1.0), (n, n_head, 2.0),
+                                             (n, n_kv, 1.0), (n, n_kv, 1.0)))]
+
+
+def assert_rows(out, ref, parts):
+    """Every row of every head by itself: |out - ref| <= (2e-6 + 2^-22 B) |A| in the 2-norm. A score of
+    magnitude up to B carries a few units of 2^-24 of B and moves its weight by as much; the weighted sums
+    and the operands' two f16 pieces (22 bits) add a few of 2^-23 of A = sum_t p_t |v_t|."""
+    a, b = parts
+    err = np.linalg.norm(out - ref, axis=2)
+    bound = (2e-6 + 2.0 ** -22 * b) * np.linalg.norm(a, axis=2)
+    bad = ~(err <= bound)
+    assert not bad.any(), (f"{int(bad.sum())} of {err.size} rows, first {np.argwhere(bad)[0]}, "
+                           f"worst {np.nanmax(err / bound):.3g}")
+
+
 PROMPT = [
     # (cache type, n_tokens, n_past, n_head, n_head_kv, head_dim, K scale, V scale): the prompt kernel's
     # tiles hold 128 (token, head of the group) rows, 32 a wave, and 32 keys a block
@@ -251,7 +292,7 @@ def test_kv_attention_prompt(KV, dev, ct, n, n_past, n_head, n_kv, hd, ks, vs):
     scale = np.float32(1.0 / (np.sqrt(hd) * ks))
     k_all = KV.gather(ct, arena_k, n_layer, layer, table, n_past, k_cur).reshape(-1, n_kv, hd)
     v_all = KV.gather(ct, arena_v, n_layer, layer, table, n_past, v_cur).reshape(-1, n_kv, hd)
-    ref, _ = KV.attention(q.reshape(n, n_head, hd), k_all, v_all, n_past, scale)
+    ref, parts = KV.attention(q.reshape(n, n_head, hd), k_all, v_all, n_past, scale)
 
     cache = dc.PagedKVCache(ct, n_blocks, n_layer, n_kv, hd, device=dev)
     cache.k.copy_(to_dev(arena_k, dev))
@@ -259,27 +300,41 @@ def test_kv_attention_prompt(KV, dev, ct, n, n_past, n_head, n_kv, hd, ks, vs):
     args = (layer, to_dev(table, dev), to_dev(q, dev), to_dev(k_cur, dev), to_dev(v_cur, dev), n_past, float(scale))
     out = to_host(cache.attention(*args)).astype(np.float64).reshape(ref.shape)
     assert np.linalg.norm(out - ref) <= 4e-6 * np.linalg.norm(ref)
+    assert_rows(out, ref, parts)  # one row of outliers does not stand in for the others
 
 
-def test_kv_attention_prompt_takes_the_splits_its_workspace_holds(KV, dev):
-    """Groups of 1 head, 96 tokens over 1500 keys: the VALU kernel's plan asked for a smaller workspace
-    than the prompt kernel's splits can use; the call runs with either and agrees to fp32 rounding."""
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("n_past,least,most", [(1500, 7, 13), (100, 1, 2)])
+def test_kv_attention_prompt_takes_the_splits_its_workspace_holds(KV, dev, n_past, least, most, hd):
+    """64 tokens of 8/2 heads: a call is accepted with the partial results of `least` key splits (1: none)
+    and told to bring those of `most`. With either, and with room between them, the result holds row by row
+    and nothing is written past the workspace; with less it is refused."""
     import torch
-    n, n_past, n_head, hd = 96, 1500, 2, 128
-    cache = dc.PagedKVCache(F16, n_past // 16 + 2, 1, n_head, hd, device=dev)
-    rows = [to_dev(synth.normal(m * n_head * hd, 40 + i).reshape(m, -1), dev)
-            for i, m in enumerate((n_past, n_past, n, n, n))]
-    table = torch.arange(n_past // 16 + 1, dtype=torch.int32, device=dev)
-    cache.write("k", 0, table, 0, rows[0])
-    cache.write("v", 0, table, 0, rows[1])
-    need = dc.kv_attention_workspace_size(n_head, n_head, hd, n, n_past)
-    outs = []
-    for nbytes in (need, 4 * need):
-        ws = torch.full((nbytes,), 255, dtype=torch.uint8, device=dev)
-        outs.append(to_host(cache.attention(0, table, *rows[2:], n_past, 0.088, workspace=ws)))
-    assert np.array_equal(outs[0], outs[1])
-    with pytest.raises(dc.DcqError):
-        cache.attention(0, table, *rows[2:], n_past, 0.088, workspace=torch.empty(256, dtype=torch.uint8, device=dev))
+    n, n_head, n_kv = 64, 8, 2
+    cache = dc.PagedKVCache(F16, n_past // 16 + 2, 1, n_kv, hd, device=dev)
+    rows = prompt_rows(hd, n_head, n_kv, n_past, n, 40)
+    table = np.random.default_rng(3).permutation(n_past // 16 + 1).astype(np.int32)
+    k_past, v_past, q, k, v = (to_dev(r, dev) for r in rows)
+    cache.write("k", 0, to_dev(table, dev), 0, k_past)
+    cache.write("v", 0, to_dev(table, dev), 0, v_past)
+    half = [KV.decode_row(F16, KV.encode_row(F16, r.reshape(-1)), r.size).reshape(r.shape) for r in rows[:2]]
+    k_all, v_all = (np.concatenate([h, c]).reshape(-1, n_kv, hd) for h, c in zip(half, rows[3:]))
+    scale = np.float32(1.0 / np.sqrt(hd))
+    ref, parts = KV.attention(rows[2].reshape(n, n_head, hd), k_all, v_all, n_past, scale)
+
+    def partials(splits):
+        o, ml = splits * n * n_head * hd * 4, splits * n * n_head * 8
+        return 0 if splits == 1 else (o + 255) // 256 * 256 + (ml + 255) // 256 * 256
+
+    assert dc.kv_attention_workspace_size(n_head, n_kv, hd, n, n_past) == partials(most)
+    for nbytes in (partials(least), partials(min(least + 2, most)) - 256, partials(most)):
+        buf = torch.full((nbytes + 4096,), 255, dtype=torch.uint8, device=dev)
+        out = to_host(cache.attention(0, to_dev(table, dev), q, k, v, n_past, float(scale), workspace=buf[:nbytes]))
+        assert_rows(out.astype(np.float64).reshape(ref.shape), ref, parts)
+        assert bool((buf[nbytes:] == 255).all())
+    if least > 1:
+        with pytest.raises(dc.DcqError):
+            cache.attention(0, to_dev(table, dev), q, k, v, n_past, float(scale), workspace=buf[:partials(least) - 256])
 
 
 @pytest.mark.parametrize("ct", [F32, F16])
@@ -305,47 +360,6 @@ def test_kv_attention_prompt_infinite_elements_leave_their_neighbours(dev, ct):
     clean, got = outs[0][:31][..., dims], outs[1][:31][..., dims]
     assert np.linalg.norm(got - clean) <= 4e-6 * np.linalg.norm(clean)
     assert not np.isfinite(outs[1][:31, :, 3]).any()
-
-
-def prompt_case(KV, dev, ct, hd, n_head, n_kv, k_past, v_past, q, k_cur, v_cur, scale, holes=()):
-    """One call over a history written to the cache (with `holes` in its block table): the output
-    [n, n_head, hd] in float64, and the oracle's (ref, (A, B)) for the same rows."""
-    n, n_past, row = q.shape[0], k_past.shape[0], n_kv * hd
-    n_blocks = (n_past + 15) // 16 + 2
-    arena_k = np.zeros(n_blocks * 16 * KV.slot_bytes(ct, row), np.uint8)
-    arena_v = np.zeros_like(arena_k)
-    table = make_table(max(n_past, 1), n_blocks, 5 + n, holes)
-    KV.write(ct, arena_k, 1, 0, table, 0, k_past)
-    KV.write(ct, arena_v, 1, 0, table, 0, v_past)
-    k_all = KV.gather(ct, arena_k, 1, 0, table, n_past, k_cur).reshape(-1, n_kv, hd)
-    v_all = KV.gather(ct, arena_v, 1, 0, table, n_past, v_cur).reshape(-1, n_kv, hd)
-    with np.errstate(invalid="ignore"):
-        ref, parts = KV.attention(q.reshape(n, n_head, hd), k_all, v_all, n_past, np.float32(scale))
-    cache = dc.PagedKVCache(ct, n_blocks, 1, n_kv, hd, device=dev)
-    cache.k.copy_(to_dev(arena_k, dev))
-    cache.v.copy_(to_dev(arena_v, dev))
-    out = cache.attention(0, to_dev(table, dev), to_dev(q, dev), to_dev(k_cur, dev), to_dev(v_cur, dev), n_past,
-                          float(scale))
-    return to_host(out).astype(np.float64).reshape(ref.shape), ref, parts
-
-
-def prompt_rows(hd, n_head, n_kv, n_past, n, seed):
-    """k_past, v_past, q, k_cur, v_cur of normal values."""
-    return [synth.normal(m * h * hd, seed + i, 0.0, std).reshape(m, h * hd)
-            for i, (m, h, std) in enumerate(((n_past, n_kv, 1.0), (n_past, n_kv, 1.0), (n, n_head, 2.0),
-                                             (n, n_kv, 1.0), (n, n_kv, 1.0)))]
-
-
-def assert_rows(out, ref, parts):
-    """Every row of every head by itself: |out - ref| <= (2e-6 + 2^-22 B) |A| in the 2-norm. A score of
-    magnitude up to B carries a few units of 2^-24 of B and moves its weight by as much; the weighted sums
-    and the operands' two f16 pieces (22 bits) add a few of 2^-23 of A = sum_t p_t |v_t|."""
-    a, b = parts
-    err = np.linalg.norm(out - ref, axis=2)
-    bound = (2e-6 + 2.0 ** -22 * b) * np.linalg.norm(a, axis=2)
-    bad = ~(err <= bound)
-    assert not bad.any(), (f"{int(bad.sum())} of {err.size} rows, first {np.argwhere(bad)[0]}, "
-                           f"worst {np.nanmax(err / bound):.3g}")
 
 
 @pytest.mark.parametrize("scale", [None, 0.0])
