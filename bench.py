@@ -8,13 +8,15 @@ Infinity Cache, so every step streams its weights from HBM. Steps are captured i
 one HIP graph (torch.cuda.CUDAGraph around the C ABI calls) and replayed, so host
 launch overhead does not enter GPU time; HIP events on the replay stream time them.
 
-Printed: one JSON line. `value` is the headline configuration's (
-Q4_K GEMV, M = 1) weight GB/s over whole steps. `roofline` is for the dominant kernel
+Printed: one JSON line. `value` is the headline configuration's (config 2: Q4_K GEMV,
+M = 1) weight GB/s over whole steps. `roofline` is for the dominant kernel
 of that step: the whole step when it is one kernel (decode with fused activation
 quantization), else the mul_mat kernel timed alone on pre-quantized activations.
-Every configuration is listed under "configs", each decode config with the measured
-pure-read time of its weight bytes (the ceiling any weight-streaming kernel can reach at
-that size) beside the 8 TB/s peak. The CPU baseline (configs 2 and 5) is a SIMD
+"configs" has each configuration's step and roofline fraction. --details writes the whole
+record to a file: every configuration, each decode config with the measured pure-read time
+of its weight bytes (the ceiling any weight-streaming kernel can reach at that size) beside
+the 8 TB/s peak, and the other workloads under "extras", whose main figures are printed to
+stderr as they are measured. The CPU baseline (configs 2 and 5) is a SIMD
 restatement of the reference CPU path (quantize once, row-partitioned AVX2 / AVX-512
 VNNI vec_dots, one pinned worker per physical core), timed on this host.
 
@@ -37,6 +39,7 @@ sys.path.insert(0, ROOT)
 METRIC = "quant mul_mat: weight GB/s at M=1, int8 TOPS at M=2048; % of MI355X roofline"
 HBM_PEAK_GBS = 8000.0     # MI355X HBM3E, 8 TB/s
 INT8_PEAK_TOPS = 5000.0   # MI355X dense int8 MFMA, 5.0 POP/s
+F16_PEAK_TFLOPS = 2500.0  # MI355X dense f16 MFMA, 2.5 PFLOP/s
 HEADLINE = 2
 
 
@@ -52,6 +55,7 @@ def parse():
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--replays", type=int, default=3)
     ap.add_argument("--no-extras", action="store_true", help="skip the gate/up pair measurement")
+    ap.add_argument("--details", metavar="FILE", help="write the whole record (all configs, extras) as JSON")
     ap.add_argument("--profile", action="store_true", help="eager steps + a calibration copy, for rocprofv3 --pmc")
     ap.add_argument("--profile-read", action="store_true",
                     help="eager pure-read launches at each config's weight size, for rocprofv3 --kernel-trace")
@@ -496,11 +500,11 @@ def bench_kv_attention(args, dev, ct, n_tokens=1, n_past=4095, n_layer=36, n_hea
                      f"n_past={n_past}, {n_layer} layers rotated",
             "us": ms * 1e3, "kernels": kern, "bytes": hist_bytes + io_bytes,
             "GBps": (hist_bytes + io_bytes) / (ms * 1e-3) / 1e9, "TFLOPs": flops / (ms * 1e-3) / 1e12,
-            # decode streams the history (HBM-bound); a long prefill is fp32 arithmetic on the VALU
+            # decode streams the history (HBM-bound); a prompt's fp32 products are three f16 MFMAs each
             "roofline": ({"bound": "hbm", "peak": 8000.0, "unit": "GB/s",
                           "frac": (hist_bytes + io_bytes) / (ms * 1e-3) / 1e9 / 8000.0} if n_tokens == 1 else
-                         {"bound": "fp32", "peak": 157.3, "unit": "TFLOP/s",
-                          "frac": flops / (ms * 1e-3) / 1e12 / 157.3})}
+                         {"bound": "f16 MFMA / 3", "peak": F16_PEAK_TFLOPS / 3, "unit": "TFLOP/s",
+                          "frac": flops / (ms * 1e-3) / 1e12 / (F16_PEAK_TFLOPS / 3)})}
 
 
 def random_weights(dev, wtype, N, K, copies, seed):
@@ -748,7 +752,7 @@ def bench_gguf_load(args, dev, mib=512):
 
 def bench_weight_quantizer(args, dev):
     """dcq_quantize_weights (ggml_quantize_chunk's algorithms on the GPU) at the weight shapes of
-    BASELINE configs 1-3 (their types), and Q4_0 / Q5_K at config 2's: ms per matrix and GB/s of
+    configs 1-3 (their types), and Q4_0 / Q5_K at config 2's: ms per matrix and GB/s of
     fp32 input (load-time work, off the hot path)."""
     import torch
     import densecore_amd as dc
@@ -797,8 +801,11 @@ def profile_config(cfg, args, dev):
 # share their kernels with configs 1 and 3 and are told apart by grid size (PROFILED below).
 PROFILE_EXTRAS = [("lm_head_q8_0_m1", "decode_q8_0_kernel", "Q8_0", 1, 151936, 1024),
                   ("lm_head_q6_k_m1", "decode_q6k_mfma_kernel", "Q6_K", 1, 151936, 2560),
-                  ("prefill_q4_k", "prefill_q4_k_kernel", "Q4_K", 2048, 8192, 2048),
-                  ("prefill_q6_k", "prefill_q6_k_kernel", "Q6_K", 2048, 8192, 2048)]
+                  ("prefill_q4_k", "gemm_kq_kernel<0,", "Q4_K", 2048, 8192, 2048),
+                  ("prefill_q6_k", "gemm_kq_kernel<2,", "Q6_K", 2048, 8192, 2048)]
+# attention calls under the same passes: (label, kernel, cache type, tokens, history, heads, KV heads, head_dim)
+PROFILE_ATTENTION = [("kv_attention_prefill_q8_0", "attn_prompt_kernel<8, 128>", "Q8_0", 2048, 0, 32, 8, 128),
+                     ("kv_attention_chunk_f16", "attn_prompt_kernel<1, 64>", "F16", 333, 2777, 32, 8, 64)]
 
 
 def profile_extras(args, dev):
@@ -818,6 +825,26 @@ def profile_extras(args, dev):
         print(f"# profiled {label}: {args.warmup + args.steps} eager calls", file=sys.stderr, flush=True)
         del big, ws, y, x
         torch.cuda.empty_cache()
+
+
+def profile_attention(args, dev):
+    """Eager calls of the PROFILE_ATTENTION shapes."""
+    import torch
+    import densecore_amd as dc
+    for label, _, tname, n, n_past, n_head, n_kv, hd in PROFILE_ATTENTION:
+        nb = (n_past + n + 15) // 16
+        cache = dc.PagedKVCache(getattr(dc, "TYPE_" + tname), nb, 1, n_kv, hd, device=dev)
+        table = torch.arange(nb, dtype=torch.int32, device=dev)
+        hist = torch.randn((max(n_past, 1), n_kv * hd), device=dev)
+        cache.write("k", 0, table, 0, hist)
+        cache.write("v", 0, table, 0, hist.roll(1, 1).contiguous())
+        q = torch.randn((n, n_head * hd), device=dev)
+        kc, vc = (torch.randn((n, n_kv * hd), device=dev) for _ in range(2))
+        for _ in range(args.warmup + args.steps):
+            cache.attention(0, table, q, kc, vc, n_past, hd ** -0.5)
+        torch.cuda.synchronize()
+        print(f"# profiled {label}: {args.warmup + args.steps} eager calls", file=sys.stderr, flush=True)
+        del cache
 
 
 def profile_read(args, dev):
@@ -925,7 +952,7 @@ def summarize_traffic(fetch_csv, write_csv):
         wt, M, N, K = shapes[label]
         algo = N * dc.row_size(wt, K) + M * K * 4 + M * N * 4
         traffic = f_kib * 1024 * fetch_scale + w_kib * 1024 * write_scale
-        lines.append(f"{label} kernel={kname} fetch_kib={f_kib:.1f} write_kib={w_kib:.1f} fetch_scale={fetch_scale:.4f} "
+        lines.append(f"{label} kernel={kname.split('<')[0]} fetch_kib={f_kib:.1f} write_kib={w_kib:.1f} fetch_scale={fetch_scale:.4f} "
                      f"write_scale={write_scale:.4f} traffic_bytes={traffic:.0f} algorithmic_bytes={algo}")
     return "\n".join(lines)
 
@@ -959,7 +986,7 @@ def summarize_pmc(paths):
             per[key][r["Counter_Name"]] = float(r["Counter_Value"])
             names[key] = (r["Kernel_Name"], int(r["Grid_Size"]))
     lines = [f"# per-dispatch medians; {agent['simds']} SIMDs, {agent['cus']} CUs, {agent['xcds']} XCDs"]
-    for label, kname, gmin, gmax in PROFILED:
+    for label, kname, gmin, gmax in PROFILED + [(f"extra={lab}", k, 0, 1 << 62) for lab, k, *_ in PROFILE_ATTENTION]:
         rows = collections.defaultdict(list)
         for key, cnt in per.items():
             if kname in names[key][0] and gmin <= names[key][1] < gmax:
@@ -970,7 +997,7 @@ def summarize_pmc(paths):
         med = {c: float(np.median(v)) for c, v in rows.items()}
         n_disp = max(len(v) for v in rows.values())
         gui = med.get("GRBM_GUI_ACTIVE")
-        kv = [label, f"kernel={kname}", f"samples={n_disp}"]
+        kv = [label, f"kernel={kname.split('<')[0]}", f"samples={n_disp}"]
         if gui:
             gui_x = gui / agent["xcds"]
             kv.append(f"gui_cycles_per_xcd={gui_x:.0f}")
@@ -1092,6 +1119,7 @@ def main():
                 profile_config(c, args, dev)
         if not args.no_extras:
             profile_extras(args, dev)
+            profile_attention(args, dev)
         calibration_copy(dev)
         return 0
     if args.profile_read:
@@ -1188,6 +1216,13 @@ def main():
                 print(f"# CPU baseline config {r['config']}: {cb['value']:.3g} {cb['unit']} on {cb['cores']} cores "
                       f"({cb['ms_per_run']:.3f} ms per run)", file=sys.stderr, flush=True)
         line["cpu_baseline"] = head.get("cpu_baseline")
+    if args.details:
+        with open(args.details, "w") as f:
+            json.dump(line, f)
+    # the line itself stays short: a reader of the output's last few thousand characters finds all of it
+    del line["extras"]
+    line["configs"] = [{"config": r["config"], "name": r["name"], "step_us": r["step_us"],
+                        "kernel_us": r["dominant_us"], "roofline_frac": r["roofline"]["frac"]} for r in results]
     print(json.dumps(line))
     return 0
 

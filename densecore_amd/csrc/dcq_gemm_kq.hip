@@ -24,11 +24,12 @@
 // has one fp32 epilogue per 16 MFMAs. iM is one f16 MFMA per tile and superblock: the activation's
 // 16-element sums are at most 2032 and the mins at most 63, both exact in f16, their products and sums
 // exact in fp32.
-// On gfx950 a wave issues about one VALU instruction per 4.7 cycles, two waves on a SIMD one per 2.5, and
-// an MFMA takes 32 cycles of its pipe and about 16 of the VALU's: 17 MFMAs (0.26 us at 2.1 GHz) and about
-// 130 VALU instructions per tile and superblock are near balance, where the per-sub-block multiply-adds
-// of the kernel before (31 VALU instructions per MFMA) were not, and its commit and barriers left half
-// the issue slots empty.
+// A SIMD issues one VALU instruction per 4 cycles at best (fma chains: 4.3 to 4.9 with two or four waves on
+// it, 5.5 to 6.2 with one), an MFMA takes 32 cycles of its pipe: per tile and superblock 17 MFMAs are 544
+// cycles and about 155 VALU instructions 620, where the kernel before had 31 VALU instructions per MFMA and
+// its commit and barriers. Counters (2048 x 8192 x 2048, Q4_K): VALU busy 45 %, MFMA 35 %, a quarter of the
+// MFMA time beside VALU, waits 38 %: neither unit is the limit, a wave's build, MFMAs and epilogue follow
+// one another and two waves a SIMD overlap little of them.
 //
 // GLU: waves 0, 1 take 64 rows of the gate matrix and waves 2, 3 the same 64 of the up matrix; at the end
 // the up waves pass their sums through LDS and the gate waves store silu(g) * u.

@@ -2,7 +2,7 @@
 //
 // A decode GEMV must stream every weight byte once, so its best possible time at a given
 // weight size is the time a kernel that does nothing but read those bytes takes. At the
-// BASELINE decode sizes (3 - 20 MB) that time is dominated by launch, ramp-up and tail, not
+// the benchmark's decode sizes (3 - 20 MB) that time is dominated by launch, ramp-up and tail, not
 // by the 8 TB/s peak, so the bench reports each decode kernel against this measured ceiling
 // beside the peak. The kernel reads `bytes` with 16-byte loads, `per_lane` loads in flight
 // per lane (all issued before any is used), 256 threads per workgroup, and folds the words

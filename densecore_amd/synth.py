@@ -1,4 +1,4 @@
-"""Deterministic synthetic inputs for the BASELINE configurations.
+"""Deterministic synthetic inputs for the benchmark's configurations.
 
 SplitMix64 (Steele, Lea, Flood 2014) feeds Box-Muller pairs; everything is
 vectorised numpy uint64/float64 arithmetic, so a seed gives the same float32

@@ -202,10 +202,11 @@ int dcq_mul_mat_noalloc(int wtype, const void* W, int64_t N, int64_t K, size_t w
  * floats; otherwise it is >= N*4. R may be Y itself (r_stride_bytes == y_stride_bytes: the
  * in-place residual) or must not overlap Y. R 4-byte aligned, strides multiples of 4; the rest
  * as dcq_mul_mat. Where the decode kernels serve the product (M <= DCQ_DECODE_ROWS(wtype, N))
- * the add is their store; otherwise the product goes to Y (or, when R is Y, a workspace
- * temporary) and one add kernel follows. workspace may
- * be NULL; otherwise it should hold dcq_mul_mat_add_workspace_size(wtype, M, N, K) bytes,
- * 256-byte aligned (the split-K room at its end is optional, as in dcq_mul_mat). */
+ * the add is their store; the K-quant GEMM adds R in its store and a split-K sum on its way
+ * out; otherwise the product goes to Y (or, when R is Y, a workspace temporary) and one add
+ * kernel follows. workspace may be NULL; otherwise it should hold
+ * dcq_mul_mat_add_workspace_size(wtype, M, N, K) bytes, 256-byte aligned (the split-K room at its
+ * end is optional, as in dcq_mul_mat). */
 size_t dcq_mul_mat_add_workspace_size(int wtype, int64_t M, int64_t N, int64_t K);
 int dcq_mul_mat_add(int wtype, const void* W, int64_t N, int64_t K, size_t w_row_bytes,
                     const float* X, int64_t M, size_t x_stride_bytes, const float* R,
@@ -332,7 +333,15 @@ int dcq_kv_gather(int cache_type, const void* arena, int64_t n_blocks, int n_lay
  * [head_dim] in fp32; query head h uses KV head h / (n_head / n_head_kv);
  * out[i][h][:] = softmax_t(scale * q . k_t) . v_t, written as [n_tokens][n_head][head_dim].
  * head_dim 64, 128 or 256; n_head a multiple of n_head_kv; n_tokens <= 65535. The workspace
- * holds per-split partial results (dcq_kv_attention_workspace_size; 0 needs none). */
+ * holds per-split partial results (dcq_kv_attention_workspace_size; 0 needs none).
+ * Precision: fp32 throughout for few query rows. From 16 rows of a KV head (n_tokens x
+ * n_head / n_head_kv; head_dim 256: 32 rows over 1024 keys) the products run on f16 matrix
+ * instructions, each fp32 operand as two f16 pieces: 22 bits or more of an element down to 2^-16 of
+ * the largest of its row (q), or of its key's row of the head (K, V), which may be up to 2^12 smaller
+ * than that of a key beside it; fewer below. Sums and softmax weights are fp32. The error against 64
+ * bits is no larger than with fp32 products (relative 2-norm 2e-7 to 5e-7). Zeros, infinities and
+ * NaN behave as in fp32 arithmetic, except that an infinite V element gives NaN, not an infinity, to
+ * a row whose weight for it is below 2^-32 of the row's largest term. */
 size_t dcq_kv_attention_workspace_size(int n_head, int n_head_kv, int head_dim, int64_t n_tokens, int64_t n_past);
 int dcq_kv_attention(int cache_type, const void* k_arena, const void* v_arena, int64_t n_blocks, int n_layer,
                      int layer, const int32_t* block_table, int64_t n_table, int n_head, int n_head_kv,

@@ -1,6 +1,6 @@
 """GPU parity: libdcq (through its C ABI) against the CPU oracle on identical inputs.
 
-Bars (BASELINE north star): quantized activation bytes and per-block int32 sums
+Bars: quantized activation bytes and per-block int32 sums
 bit-exact; fp32 outputs within |y - y_ref| <= 1e-4 * max(|y_ref|, L1), where L1
 is the sum of the magnitudes of the fp32 terms the reference adds (|scale_b * int_b|
 per Q8_0 / Q4_0 block; the eight per-superblock lane sums of Q4_K / Q5_K / Q6_K, plus the mins
@@ -337,7 +337,7 @@ def test_dequantize_rows(O, dev, wt):
     np.testing.assert_allclose(got, want, rtol=2e-7, atol=0)
 
 
-# ---------------------------------------------------------------- BASELINE configurations
+# ---------------------------------------------------------------- the benchmark's configurations
 @pytest.mark.parametrize("cfg", dc.CONFIGS, ids=lambda c: f"cfg{c.index}")
 def test_baseline_config_parity(O, dev, cfg):
     """Full-size configs, every output against the oracle (config 5: all 2048 x 8192 outputs, so
