@@ -96,6 +96,11 @@ ATTN = [
     # per row)
     (Q8_0, 1, 2000, 32, 8, 128),   # 33 splits
     (Q8_0, 1, 7000, 32, 8, 128),   # 111 splits
+    (Q8_0, 1, 300, 32, 8, 128),    # 6 splits of 1024 quads: lanes
+    (Q8_0, 1, 500, 32, 8, 128),    # 9 splits
+    (F16, 16, 600, 16, 1, 64),     # 6 splits of 4096 quads
+    (F16, 33, 700, 16, 2, 64),     # 7 splits of 8448 quads: a thread per quad
+    (F16, 34, 1300, 16, 2, 128),   # more of them
     (F16, 1, 20000, 4, 4, 64),     # 158 splits
     (F16, 5, 33, 16, 4, 64),
     (F32, 1, 200, 8, 2, 128),
