@@ -860,19 +860,40 @@ static AttnPlan attn_plan(int hd, int n_head, int n_head_kv, int n_tokens, int n
     return p;
 }
 
+// Workgroups of a VALU plan's launch (key splits in eights, one XCD each).
+static int64_t attn_wgs(const AttnPlan& p) {
+    return (int64_t)(p.splits > 1 ? (p.splits + 7) / 8 * 8 : 1) * p.groups * p.qtiles;
+}
+
 // Prompts and prompt chunks take the MFMA kernel (dcq_attn_prompt.hip) from 16 query rows of a KV head
-// (tokens x the query heads of its group); at head_dim 256, where a workgroup fills a CU and a block
-// takes longer, from 32 rows over 1024 keys. Per call, VALU kernel -> MFMA kernel (us, MI355X):
-//   8 KV heads x 128, groups of 4, Q8_0: 16 rows over 0 / 300 / 4096 keys 12.7 -> 7.3, 19.2 -> 15.7,
-//   31.3 -> 17.8 (8 rows: 8.2 -> 7.2, 13.7 -> 15.7, 20.7 -> 16.8); 2 KV heads x 128, groups of 8, F32: 16
-//   rows 12.5 -> 6.9, 17.2 -> 15.2, 17.0 -> 16.0; 4 KV heads x 64, groups of 7, F16: 14 rows 11.4 -> 5.1,
-//   15.7 -> 11.7, 15.9 -> 12.4
-//   4 KV heads x 256, groups of 2, Q8_0: 32 rows over 4096 keys 52.1 -> 31.7, 64 rows 82.7 -> 37.3; but
-//   128 rows over 300 31.6 -> 35.6 and a 128-token prompt 23.3 -> 33.9
-static bool attn_use_prompt(int hd, int n_head, int n_head_kv, int n_tokens, int n_past) {
-    const int64_t rows = (int64_t)n_tokens * (n_head / n_head_kv);
-    if (n_tokens < 2 || knob(Knob::AttnNoMfma) != 0) return false;
-    return hd < 256 ? rows >= 16 : rows >= 32 && n_past + n_tokens >= 1024;
+// (tokens x the query heads of its group), but for calls that the VALU kernel does in few rounds of
+// workgroups. Per call, VALU kernel -> MFMA kernel (us, MI355X, graphs of 10 to 20 calls; 64 to 8192 keys,
+// 16 to 512 rows, 1 to 8 KV heads):
+//   x 64: always faster, 0.48 to 0.93 of the VALU kernel's time
+//   x 128: 16 rows of 8 KV heads, Q8_0, over 0 / 300 / 4096 keys 12.9 -> 9.3, 19.2 -> 15.4, 32.5 -> 19.7 (8 rows:
+//   8.2 -> 7.2, 13.7 -> 15.7). More than 64 rows over 200 keys or more are the VALU kernel's while its workgroups
+//   are at most two per CU (Q8_0, which it decodes through LDS: one): 133 rows of 2 KV heads, F16, over 384 keys
+//   17.8 -> 19.9, over 1000 18.6 -> 21.7; over 1500, 608 workgroups, 26 -> 19. Calls of 32 tokens with groups of 4k
+//   heads stay on the MFMA kernel there (up to 17 % slower): they are accepted with less workspace than the
+//   VALU kernel's splits need
+//   x 256, where a block takes the MFMA kernel longest: 32 rows and 1024 keys or more, from 5 chunks one after
+//   another (chunks per split x rounds of 3 workgroups per CU), Q8_0 from 2 chunks per split. 8 tokens of 4/1
+//   heads over 1016 keys, F32, 13.3 -> 34.1; 16 of 32/8 over 1014, F16, 6 chunks, 49 -> 34.5; 64 of 4/1 over 2236, 3
+//   chunks, 31.4 -> 37.2; Q8_0 at 2 chunks per split 0.68 to 1.01 of the VALU kernel's time, at 1 0.91 to 2.1
+static bool attn_use_prompt(int ct, int hd, int n_head, int n_head_kv, int n_tokens, int n_past) {
+    const int rep = n_head / n_head_kv;
+    const int64_t rows = (int64_t)n_tokens * rep, keys = (int64_t)n_past + n_tokens, cus = cu_count();
+    const bool q8 = ct == kTypeQ8_0;
+    if (n_tokens < 2 || rows < 16 || knob(Knob::AttnNoMfma) != 0) return false;
+    if (hd == 64 || (hd == 128 && (rows <= 64 || keys < 200 || (n_tokens >= 32 && rep % 4 == 0)))) return true;
+    const AttnPlan p = attn_plan(hd, n_head, n_head_kv, n_tokens, n_past);
+    if (hd == 128) return attn_wgs(p) > (q8 ? cus : 2 * cus);
+    if (rows < 32 || keys < 1024) return false;
+    return q8 ? p.cps >= 2 : p.cps * ((attn_wgs(p) + 3 * cus - 1) / (3 * cus)) >= 5;
+}
+// Whether some cache type's call does (Q8_0's do first): the workspace query does not know the type.
+static bool attn_may_use_prompt(int hd, int n_head, int n_head_kv, int n_tokens, int n_past) {
+    return attn_use_prompt(kTypeQ8_0, hd, n_head, n_head_kv, n_tokens, n_past);
 }
 
 // Bytes of the key splits' partial results: O [splits][tokens][heads][hd], then (m, l).
@@ -908,8 +929,8 @@ static PromptPlan attn_prompt_plan(int hd, int n_head, int n_head_kv, int n_toke
 // first prompt kernel (groups of 4k heads, head_dim 64 or 128, 32 tokens) 32-token tiles of 4 heads.
 // attn_workspace_bytes may ask for more, which the prompt kernel's splits use when they find it.
 size_t attn_workspace_min_bytes(int hd, int n_head, int n_head_kv, int n_tokens, int n_past) {
-    if (attn_use_prompt(hd, n_head, n_head_kv, n_tokens, n_past) && (hd == 64 || hd == 128) && (n_head / n_head_kv) % 4 == 0 &&
-        n_tokens >= 32) {
+    if (attn_may_use_prompt(hd, n_head, n_head_kv, n_tokens, n_past) && (hd == 64 || hd == 128) &&
+        (n_head / n_head_kv) % 4 == 0 && n_tokens >= 32) {
         const int64_t base = (int64_t)((n_tokens + 31) / 32) * (n_head / 4);
         const int nblk = (n_past + n_tokens + 31) / 32;
         const int64_t want = std::max<int64_t>(1, std::min<int64_t>((512 + base - 1) / base, (nblk + 7) / 8));
@@ -921,7 +942,7 @@ size_t attn_workspace_min_bytes(int hd, int n_head, int n_head_kv, int n_tokens,
 
 size_t attn_workspace_bytes(int hd, int n_head, int n_head_kv, int n_tokens, int n_past) {
     const size_t least = attn_workspace_min_bytes(hd, n_head, n_head_kv, n_tokens, n_past);
-    if (!attn_use_prompt(hd, n_head, n_head_kv, n_tokens, n_past)) return least;
+    if (!attn_may_use_prompt(hd, n_head, n_head_kv, n_tokens, n_past)) return least;
     const PromptPlan m = attn_prompt_plan(hd, n_head, n_head_kv, n_tokens, n_past, SIZE_MAX);
     return std::max(least, attn_partial_bytes(m.splits, hd, n_head, n_tokens));
 }
@@ -974,7 +995,7 @@ hipError_t launch_kv_attention(int ct, const void* k_arena, const void* v_arena,
                                const float* q, int64_t q_stride, const float* k_cur, const float* v_cur,
                                int64_t kv_stride, int n_tokens, int n_past, float scale, float* out,
                                int64_t out_stride, void* ws, size_t ws_bytes, hipStream_t st) {
-    const bool prompt = attn_use_prompt(hd, n_head, n_head_kv, n_tokens, n_past);
+    const bool prompt = attn_use_prompt(ct, hd, n_head, n_head_kv, n_tokens, n_past);
     const AttnPlan p = attn_plan(hd, n_head, n_head_kv, n_tokens, n_past);
     if (ws_bytes < attn_workspace_min_bytes(hd, n_head, n_head_kv, n_tokens, n_past)) return hipErrorInvalidValue;
     AttnArgs a{};
@@ -1003,7 +1024,7 @@ hipError_t launch_kv_attention(int ct, const void* k_arena, const void* v_arena,
         return launch_attn_combine(a.ws_o, a.ws_ml, m.splits, n_tokens, n_head, hd, out, out_stride, st);
     }
     if (p.splits > 1) partials(p.splits);
-    const int64_t wgs = (int64_t)(p.splits > 1 ? (p.splits + 7) / 8 * 8 : 1) * p.groups * p.qtiles;
+    const int64_t wgs = attn_wgs(p);
     if (wgs > INT32_MAX) return hipErrorInvalidValue;
     const dim3 grid((unsigned)wgs);
 #define DCQ_ATTN_CASE(C, H)           \

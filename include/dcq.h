@@ -335,8 +335,8 @@ int dcq_kv_gather(int cache_type, const void* arena, int64_t n_blocks, int n_lay
  * head_dim 64, 128 or 256; n_head a multiple of n_head_kv; n_tokens <= 65535. The workspace
  * holds per-split partial results (dcq_kv_attention_workspace_size; 0 needs none).
  * Precision: fp32 throughout for few query rows. From 16 rows of a KV head (n_tokens x
- * n_head / n_head_kv; head_dim 256: 32 rows over 1024 keys) the products run on f16 matrix
- * instructions, each fp32 operand as two f16 pieces: 22 bits or more of an element down to 2^-16 of
+ * n_head / n_head_kv; at head_dim 128 and 256 where there is more work than fp32 does in about the
+ * same time) the products run on f16 matrix instructions, each fp32 operand as two f16 pieces: 22 bits or more of an element down to 2^-16 of
  * the largest of its row (q), or of its key's row of the head (K, V), which may be up to 2^12 smaller
  * than that of a key beside it; fewer below. Sums and softmax weights are fp32. The error against 64
  * bits is no larger than with fp32 products (relative 2-norm 2e-7 to 5e-7). Zeros, infinities and

@@ -262,15 +262,20 @@ PROMPT = [
     (F32, 129, 0, 2, 2, 64, 1, 1),         # one row past a tile, no history
     (F16, 43, 31, 12, 4, 128, 1, 1),       # groups of 3 (129 rows): tokens straddle waves and tiles
     (Q8_0, 19, 290, 28, 4, 64, 1, 1),      # groups of 7, the keys split over workgroups
-    (F16, 64, 960, 4, 2, 256, 1, 1),       # head_dim 256, exact blocks and tiles, the fewest keys
+    (F16, 64, 960, 4, 2, 256, 1, 1),       # head_dim 256 in few rounds: the VALU kernel
     (Q8_0, 33, 990, 8, 8, 256, 1, 1),      # 33 rows over 1023 keys: the VALU kernel
-    (F32, 9, 1300, 8, 1, 256, 1, 1),       # 72 rows, the keys split
+    (F32, 9, 1300, 8, 1, 256, 1, 1),
     (F32, 70, 20, 4, 1, 128, 3e-7, 2e5),   # magnitudes past f16's range on either side
     (F32, 70, 20, 4, 1, 64, 1e-20, 1e20),
     (F32, 200, 0, 4, 1, 128, 1, 1e-12),
     (F16, 40, 24, 4, 1, 128, 1, 1),        # two blocks: one for each wave group
     (Q8_0, 90, 700, 6, 2, 128, 1, 1),      # key splits with odd numbers of blocks
     (F32, 700, 0, 3, 1, 64, 1, 1),         # a causal prompt with key splits that early tiles do not reach
+    (F16, 64, 2752, 4, 2, 256, 1, 1),      # head_dim 256, past the VALU kernel's few rounds: exact blocks and tiles
+    (Q8_0, 64, 1153, 4, 2, 256, 1, 1),     # Q8_0 earlier
+    (F32, 9, 8400, 8, 1, 256, 1, 1),       # 72 rows, the keys split
+    (Q8_0, 19, 300, 14, 2, 128, 1, 1),     # 133 rows, few workgroups of the VALU kernel: that one
+    (Q8_0, 19, 1500, 14, 2, 128, 1, 1),    # ... and more of them: the prompt kernel
 ]
 
 
@@ -373,8 +378,8 @@ def test_kv_attention_prompt_infinite_elements_leave_their_neighbours(dev, ct):
     (F16, 56, 0, 4, 2, 128),      # 24: one padded group of 8 keys
     (Q8_0, 40, 17, 4, 1, 64),     # 25: no padded group
     (F32, 48, 16, 2, 1, 128),     # 0: no padding
-    (F16, 19, 1021, 4, 1, 128),   # 16, the keys split over workgroups
-    (Q8_0, 20, 1005, 8, 1, 256),  # 1, split
+    (F16, 16, 1024, 4, 1, 128),   # 16, the keys split over workgroups
+    (Q8_0, 20, 3757, 8, 1, 256),  # 1, split
     (F32, 160, 1200, 16, 8, 256),  # 16, many tiles
 ])
 def test_kv_attention_prompt_zero_rows(KV, dev, ct, n, n_past, n_head, n_kv, hd, scale):
@@ -390,7 +395,7 @@ def test_kv_attention_prompt_zero_rows(KV, dev, ct, n, n_past, n_head, n_kv, hd,
 
 @pytest.mark.parametrize("past,cur", [(0.0, 1.0), (0.0, 1e25), (0.0, 1e-30), (1e-30, 1.0), (1.0, 1e30), (1e30, 1e-30),
                                       (1e-4, 1.0), (1e-36, 1e-36), (1e35, 1e36)])
-@pytest.mark.parametrize("n_past,hd", [(300, 64), (300, 128), (1030, 256)])
+@pytest.mark.parametrize("n_past,hd", [(300, 64), (300, 128), (3800, 256)])
 def test_kv_attention_prompt_value_magnitudes(KV, dev, n_past, hd, past, cur):
     """Values of one magnitude in the history and another in the batch: no key's weight is lost from
     the sum of weights, whatever its values are beside the others'."""
@@ -400,7 +405,7 @@ def test_kv_attention_prompt_value_magnitudes(KV, dev, n_past, hd, past, cur):
 
 
 @pytest.mark.parametrize("n_kv,hd", [(512, 64), (256, 128), (256, 256),  # a workgroup per CU: the keys unsplit
-                                     (2, 64), (2, 128), (2, 256)])       # the keys split
+                                     (2, 64), (2, 128), (4, 256)])       # the keys split
 def test_kv_attention_prompt_missing_history(dev, n_kv, hd):
     """8200 history positions without a block read as zero rows: score 0, value 0, in the sum of weights."""
     import torch
@@ -424,11 +429,11 @@ def test_kv_attention_prompt_missing_history(dev, n_kv, hd):
 
 
 @pytest.mark.parametrize("bits", [10, 20, 30, 40])
-@pytest.mark.parametrize("n_past,hd", [(41, 64), (300, 128), (1040, 256)])
+@pytest.mark.parametrize("n_past,hd", [(41, 64), (300, 128), (2040, 256)])
 def test_kv_attention_prompt_outlier_keys(KV, dev, n_past, hd, bits):
     """A key 2^bits times its neighbours, hidden from a row (a later token) or of no weight for it, costs
     the keys staged beside it no bits: each row by itself."""
-    n, n_kv, n_head = 37, 2, 6
+    n, n_kv, n_head = 37, 2, 8
     k_past, v_past, q, k_cur, v_cur = prompt_rows(hd, n_head, n_kv, n_past, n, 600 + bits)
     big = np.float32(2.0 ** bits)
     q.reshape(n, n_head, hd)[:, :, 5] = 2.0
@@ -443,7 +448,7 @@ def test_kv_attention_prompt_outlier_keys(KV, dev, n_past, hd, bits):
 
 
 @pytest.mark.parametrize("ct", [F32, F16])
-@pytest.mark.parametrize("hd,n_past", [(64, 40), (128, 300), (256, 1001)])
+@pytest.mark.parametrize("hd,n_past", [(64, 40), (128, 300), (256, 3130)])
 def test_kv_attention_prompt_infinities(KV, dev, ct, hd, n_past):
     """As in fp32 arithmetic: a score of minus infinity has no weight, one of plus infinity makes its row
     NaN, and an infinite value makes its dim infinite for the rows that see it, and leaves the others."""
@@ -468,7 +473,7 @@ def test_kv_attention_prompt_infinities(KV, dev, ct, hd, n_past):
 
 @pytest.mark.parametrize("ct,n,n_past,n_head,n_kv,hd", [
     (Q8_0, 4, 4095, 32, 8, 128), (F32, 2, 8000, 16, 2, 128), (Q8_0, 8, 1000, 28, 4, 128), (F32, 21, 3000, 7, 1, 64),
-    (Q8_0, 8, 4000, 16, 4, 256), (F32, 40, 1500, 4, 2, 256), (F16, 150, 900, 4, 2, 256)])
+    (Q8_0, 8, 4800, 16, 4, 256), (F32, 40, 3800, 4, 2, 256), (F16, 150, 900, 4, 2, 256)])
 def test_kv_attention_prompt_precision(KV, dev, ct, n, n_past, n_head, n_kv, hd):
     """Shapes that the VALU kernel would serve in fp32: its relative 2-norm error on them is 3.6e-7 to 4.6e-7,
     that of one chain of MFMAs for all of a score's products 4.9e-7 to 9.0e-7. At most 5e-7."""
