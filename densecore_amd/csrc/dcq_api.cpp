@@ -470,7 +470,7 @@ int dcq_ffn_gate_up(int wtype, const void* Wg, const void* Wu, int64_t N, int64_
     const SplitScratch sc = tail_of(ws, workspace ? workspace_bytes : need, act_bytes + (size_t)M * N * 4);
     hipError_t e = launch_quantize_planar(vdt, X, (int64_t)(x_stride_bytes / 4), M, K, pb, st);
     const bool use_gemv = M <= gemv_rows(wtype, N, K, false);
-    if (e == hipSuccess && !use_gemv && gemm_kq_wins(wtype, M, N, K, true)) {
+    if (e == hipSuccess && !use_gemv && gemm_kq_wins(wtype, M, N, K, true, sc)) {
         // one kernel: gate and up tiles in one workgroup, their product its store
         e = launch_gemm_kq(wtype, Wg, Wu, (int64_t)w_row_bytes, N, K, pb, M, Y, y_stride, st);
         if (e != hipErrorNotSupported) {

@@ -477,25 +477,39 @@ static GemmPlan plan_gemm(int wtype, int64_t M, int64_t N, int bn, int nsb, bool
 //     1024 49.8 -> 28.4, Q5_K 59.2 -> 42.4, Q6_K 75.9 -> 49.3; 16 x 32768 x 1792 17.8 -> 16.4, but Q5_K 20.3 against
 //     21.4
 //   Q6_K rows of an odd number of superblocks, which only the generic kernel takes: 1000 x 9728 x 2816 469 -> 119,
-//     64 x 2560 x 9472 111 -> 30.0, 33 x 1024 x 1280 22.2 -> 18.5; but 16 x 4096 x 2816 21.5 against 24.8
+//     64 x 2560 x 9472 111 -> 30.0, 33 x 1024 x 1280 22.2 -> 18.5; but 16 x 4096 x 2816 21.5 against 24.8, 33 x 1024 x
+//     1792 24.2 against 26.3, and without room to split K (the generic kernel's waves split it) 5 x 2048 x 11008 54
+//     against 138, 192 x 2048 x 7936 77 against 102, while 192 x 4096 x 7936 102 and 103, 512 x 4096 x 7936 222 -> 109
 // Gate/up pairs (against two products and the SiLU kernel):
 //   Q4_K, Q5_K: 2048 x 9728 x 2560 345 -> 279 (Q5_K 355 -> 321), 256 x 4096 x 4096 48.1 -> 41.0, 72 x 8192 x 2048
 //     30.7 -> 22.2, 16 x 9728 x 2560 21.9 -> 19.1; but 128 x 4096 x 4096 27.1 against 28.9, 64 x 4096 x 4096 20.3
 //     against 27.9, Q5_K 16 x 9728 x 2560 25.1 against 26.0
 //   Q6_K: 2048 x 9728 x 2560 396 -> 318, 72 x 8192 x 2048 35.5 -> 30.0, 512 x 1024 x 2560 41.7 -> 30.8, 48 x 9728 x
 //     2560 48.6 -> 36.4; but 128 x 4096 x 4096 37.3 against 47.7, 32 x 9728 x 2560 31.3 against 31.6
-bool gemm_kq_wins(int wtype, int64_t M, int64_t N, int64_t K, bool glu) {
+//   Long rows of few tiles, where the two products split K and the pair cannot: Q6_K 512 x 1024 x 13824 78 against
+//     143, 1200 x 1024 x 6144 86 against 107, 160 tiles x 16 superblocks 69 against 76, but 1200 x 2048 x 6144 177 -> 148,
+//     256 x 4096 x 4096 58 -> 54; Q5_K 600 x 256 x 6144 50 against 57, 1200 x 512 x 13824 117 against 133; Q4_K 600 x
+//     256 x 13824 63 against 75
+bool gemm_kq_wins(int wtype, int64_t M, int64_t N, int64_t K, bool glu, const SplitScratch& sc) {
     if ((wtype != kTypeQ4_K && wtype != kTypeQ5_K && wtype != kTypeQ6_K) || M <= 4) return false;
     if (knob(Knob::GemmKq) >= 0) return knob(Knob::GemmKq) != 0;
     const int64_t nsb = K / 256;
-    if (wtype == kTypeQ6_K && nsb % 2 && (M > 32 || N * K >= (int64_t)1 << 24)) return true;
+    if (wtype == kTypeQ6_K && nsb % 2) {
+        const bool split = !glu && nsb >= 8 && sc.p && sc.bytes >= (size_t)(2 * M * N) * sizeof(float);
+        if (M <= 32) return split && nsb >= 11 && N * K >= (int64_t)1 << (nsb >= 13 ? 24 : 25);
+        if (glu || nsb <= 5 || (M <= 64 && N >= 16384 && nsb <= 16)) return true;
+        if (split && (nsb >= 11 || M > 48)) return true;
+        return M * N >= (nsb <= 16 ? 600000 : 800000);
+    }
     if (glu) {
         if (wtype == kTypeQ6_K) {
             const int64_t tiles = (M + 127) / 128 * ((N + 63) / 64);
-            return M > 32 && tiles >= (M > 256 ? 64 : 128);
+            if (M <= 32 || tiles < (M > 256 ? 64 : 128)) return false;
+            return M <= 64 || nsb <= 12 || tiles >= 192 || (nsb <= 16 && tiles >= 96 && tiles <= 128);
         }
         if (M <= 64) return N >= 9216 && (M > 32 || wtype == kTypeQ4_K);
-        return M > 512 || N >= 8192 || M * N >= 1000000;
+        if (M > 512) return wtype == kTypeQ4_K ? nsb <= 24 || M * N >= 250000 : nsb <= 16 || M * N >= 700000;
+        return N >= 8192 || M * N >= 1000000;
     }
     if (M <= 32) return nsb < 8 && N >= (wtype == kTypeQ5_K ? 65536 : 32768);
     if (M <= 64) return N >= 25600;

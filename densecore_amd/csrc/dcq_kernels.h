@@ -179,8 +179,9 @@ hipError_t launch_prefill_q4_k(bool q5, const void* W, int64_t w_row_bytes, int6
 hipError_t launch_gemm_kq(int wtype, const void* W, const void* W2, int64_t w_row_bytes, int64_t N, int64_t K,
                           const PlanarBuffers& act, int64_t M, float* Y, int64_t y_stride, hipStream_t st,
                           const SplitScratch& sc = SplitScratch());
-// Whether launch_gemm_kq is the faster kernel for a product (glu: a gate/up pair); false for other types.
-bool gemm_kq_wins(int wtype, int64_t M, int64_t N, int64_t K, bool glu);
+// Whether launch_gemm_kq is the faster kernel for a product (glu: a gate/up pair) with the room of sc to split K;
+// false for other types.
+bool gemm_kq_wins(int wtype, int64_t M, int64_t N, int64_t K, bool glu, const SplitScratch& sc);
 
 // Q4_K (q5: Q5_K) batched decode (M <= 128): 8-wave workgroups per 32 weight rows x 64 activation
 // rows, K split over the waves (and over workgroups when the rows are few and sc has room);

@@ -609,7 +609,7 @@ hipError_t launch_mmq(int wtype, const void* W, int64_t w_row_bytes, int64_t N, 
     // 25.5 -> 33.3 us, and at K >= 8192 from 128 rows)
     const bool batch_past_64 =
         M <= 256 && K <= 4096 && ((N + 31) / 32) * ((M + 63) / 64) <= (int64_t)cu_count();
-    if (gemm_kq_wins(wtype, M, N, K, false) && !block_sums) {
+    if (gemm_kq_wins(wtype, M, N, K, false, sc) && !block_sums) {
         const hipError_t e = launch_gemm_kq(wtype, W, nullptr, w_row_bytes, N, K, act, M, Y, y_stride, st, sc);
         if (e != hipErrorNotSupported) return e;
     }

@@ -752,7 +752,8 @@ def test_batch_small_m(O, dev, wt, M, N, K):
 # sends a product to it (past 512 rows, tall matrices, few superblocks, an odd number of them for Q6_K).
 GEMM_KQ = [(Q4_K, 513, 97, 256), (Q5_K, 641, 130, 768), (Q4_K, 142, 9217, 256), (Q5_K, 16, 65537, 256),
            (Q4_K, 5, 32768, 512), (Q6_K, 40, 70, 768), (Q6_K, 129, 16390, 512), (Q6_K, 5, 65537, 256),
-           (Q6_K, 33, 1, 1280), (Q5_K, 33, 25600, 256), (Q4_K, 600, 128, 4096), (Q6_K, 100, 200, 2816)]
+           (Q6_K, 33, 1, 1280), (Q5_K, 33, 25600, 256), (Q4_K, 600, 128, 4096), (Q6_K, 100, 200, 2816),
+           (Q6_K, 24, 5050, 3328), (Q6_K, 75, 8001, 1792)]
 
 
 @pytest.mark.parametrize("wt,M,N,K", GEMM_KQ)
